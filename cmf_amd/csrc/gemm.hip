@@ -3,21 +3,29 @@
 // Y[b][n] = sum_k X[b][k] W[n][k] for b < M (any M), W in the q4t / q4tp
 // device layout of the GEMV kernels.
 //
-// Tiling (MFMA f32 16x16x32 f16): a workgroup of 4 waves owns 64 batch rows
-// x 64 GRB weight rows (wave w holds GRB row blocks in registers), and walks
-// K in steps of 128 columns (4 tiles):
-//   - the operand step (hi / lo f16 planes of 64 rows x 4 tiles and their
-//     two tables of tile biases, 34 KiB) is loaded into registers one step ahead and
-//     written to the other half of a double-buffered LDS tile after the
-//     current step's MFMAs (one barrier per step);
-//   - the weights of the next step (4 row blocks x 1 KiB + scales per wave)
-//     are requested before the current step is computed;
-//   - per tile and row block: the nibbles become f16 denormals n * 2^-24
-//     (one mask per pair); the hi and lo planes (fixed point, prep16_row)
-//     take one MFMA each, each started at its plane's tile bias
-//     -8 * 2^-24 * sum (so D = 2^-24 * sum((n - 8) x) / xs exactly), and the
-//     tile scale multiplies D in f32 as q4t_row_exact does
-//     (qtensor.rs:4418-4432).
+// Tiling (MFMA f32 32x32x16 f16): a workgroup of 4 waves owns 64 batch rows
+// x 128 RN weight rows (wave w holds 32 RN of them) and walks K in stages of
+// two tiles (64 columns):
+//   - a stage's operand (hi / lo f16 planes of 64 rows, 16 KiB) goes straight
+//     from global memory into one of three LDS slots, two stages ahead;
+//   - the weights and scales of the next group of four tiles are requested
+//     into registers a group ahead, each wave its own rows;
+//   - the nibbles become the f16 integers n - 8 (dq_signed), so a tile needs
+//     no bias; a block of 32 x 32 outputs takes four MFMAs per tile, the lo
+//     plane's two and then the hi plane's two in one accumulator started at
+//     zero: the lo sum is exact, the hi products are integers, and the one
+//     rounding of their sum is that of the f32 add it replaces (measured on
+//     K = 4096: 2.06e-7 from an f64 product with one accumulator, 2.05e-7
+//     with two and an add); the tile scale multiplies the sum in f32 as
+//     q4t_row_exact does (qtensor.rs:4418-4432).
+// Bound by issue: per tile and block 4 MFMAs (128 cycles of the matrix
+// pipe) stand beside 16 FMAs (the tile scale) and 9 VALU ops that unpack
+// weights (100 cycles), and the clock falls to ~1.85 GHz under this load.
+// Measured on MI355X, operand preparation included: q4t 12288x4096 m = 2048
+// 571 -> 402 us, 6144x1024 123 -> 81, 1024x3072 91 -> 65, 12288x4096 m = 256
+// 123 -> 87, m = 64 57 -> 42; q4tp 12288x4096 m = 2048 891 -> 410 (the
+// 16x16x32 form with an accumulator per plane and tile biases from LDS took
+// 8 FMAs and adds per two MFMAs, and as many LDS as matrix cycles).
 #include <mutex>
 #include <set>
 
@@ -30,7 +38,7 @@ struct GemmArgs {
     const void* w;        // [rb][group of 4 tiles][lane][16 B]   (q8: [rb][64-column chunk][lane][16 B])
     const void* scale;    // q4t f16 [rb][group][16][4]; q4tp u32 codes; q8 f32 row scales
     const float2* rowp;   // q4tp (2^lo, 2^step) per row
-    const uint8_t* planes;  // hi [item][Mp], lo [item][Mp] (16 B), biases hi / lo [tile][Mp] f32 (q8: q0 q1 q2 [item][Mp])
+    const uint8_t* planes;  // hi [item][Mp], lo [item][Mp] (16 B) (q8: q0 q1 q2 [item][Mp])
     const float* xs;      // [Mp] 2^-e per batch row (q8: amax / 127)
     float* y;
     int ldy, M, Mp, N, ntg, nrb, resid;
@@ -41,195 +49,239 @@ struct GemmArgs {
     float* part;
 };
 
+constexpr int G4_NB = 3;           // k_gemm_q4: operand stages in LDS
+constexpr size_t GEMM_AT_BYTES = (size_t)G4_NB * 16 * 1024;  // its dynamic LDS
 constexpr int GB = 64;             // batch rows per workgroup
-constexpr int GCH = 34;            // 1 KiB operand chunks per K step (16 hi + 16 lo items, hi and lo biases)
-constexpr int GJ = (GCH + 3) / 4;  // chunks per wave (clamped)
-// k_gemm_q4's dynamic LDS: the operand tile [2][GCH][64] x 16 B, then the
-// weight rows' tile scales [2][4 waves] x 1 KiB
-constexpr size_t GEMM_AT_BYTES = (size_t)2 * GCH * 64 * 16 + (size_t)2 * 4 * 1024;
 
 // s_waitcnt lgkmcnt(0) + s_barrier: an LDS-only workgroup barrier (the
 // weight loads in flight are not waited for, as __syncthreads would)
 __device__ __forceinline__ void lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// GRB: row blocks per wave (4 for large batches; 1 gives small batches 4x
-// the workgroups).
-template <int FMT, int GRB>
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t uint4r __attribute__((ext_vector_type(4)));
+
+// Four nibble bytes as the f16 integers n - 8, in-slot order
+// {0,4,2,6,1,5,3,7}: a nibble or-ed into 1024.0's mantissa is 1024 + n (low
+// nibble of a byte) or 1024 + 16 n (high nibble); both become n - 8 exactly
+// by one packed f16 op.
+__device__ __forceinline__ half8 dq_signed(uint32_t w) {
+    constexpr uint32_t LO = 0x000F000Fu, HI = 0x00F000F0u, M = 0x64006400u;
+    const half2v k1 = {(_Float16)-1032.f, (_Float16)-1032.f}, k2 = {(_Float16)0.0625f, (_Float16)0.0625f},
+                 k3 = {(_Float16)-72.f, (_Float16)-72.f};
+    const uint32_t w8 = w >> 8;
+    auto mo = [](uint32_t x, uint32_t mask) __attribute__((always_inline)) {
+        uint32_t y;  // (x & mask) | M, one instruction: the mask an SGPR, M a VGPR
+        asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(y) : "v"(x), "s"(mask), "v"(M));
+        return __builtin_bit_cast(half2v, y);
+    };
+    const half2v a = mo(w, LO) + k1;    // elements 0, 4
+    const half2v b = mo(w8, LO) + k1;   // 2, 6
+    const half2v c = __builtin_elementwise_fma(mo(w, HI), k2, k3);   // 1, 5
+    const half2v d = __builtin_elementwise_fma(mo(w8, HI), k2, k3);  // 3, 7
+    return half8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+// RN: 32-row weight blocks per wave.
+template <int FMT, int RN>
 __global__ __launch_bounds__(256, 2) void k_gemm_q4(GemmArgs a) {
     constexpr bool TP = FMT == DT_Q4TP;
-    // the double-buffered operand tile [2][GCH chunks][64 lanes] x 16 B,
-    // filled by direct global -> LDS loads (dynamic LDS: with a static array
-    // as the load target the compiler waits for every load in flight before
-    // each LDS read)
+    constexpr int MB = 2, BM = GB;  // 32-row batch blocks, batch rows per workgroup
+    constexpr int TPS = 2;          // tiles per stage (a stage's operand: 16 KiB)
+    constexpr int SPG = 4 / TPS;    // stages per group of 4 tiles
+    constexpr int NB = G4_NB;       // operand stages in LDS
+    constexpr int NCH = 4;         // 1 KiB operand chunks per wave and stage
+    constexpr int NW = 3 * RN;     // weight and scale loads per group
+    // the operand ring [NB][plane][4 TPS items][BM rows] x 16 B, filled by
+    // direct global -> LDS loads (dynamic LDS: with a static array as the
+    // load target the compiler waits for every load in flight before each
+    // LDS read)
     extern __shared__ __align__(16) uint4 gemm_at[];
-    __shared__ float lad[TP ? 4 : 1][TP ? GRB * 16 * 33 : 1];
+    // q4tp: the 32 rungs of every row, rung c of row i in word c ^ (i % 32)
+    // (rows' equal rungs in different banks)
+    __shared__ float lad[TP ? 4 * RN * 32 * 32 : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, s = lane >> 4;
-    const int by = blockIdx.y, rbw = (blockIdx.x * 4 + wave) * GRB;  // first row block of this wave
+    const int c32 = lane & 31, h = lane >> 5, r = lane & 15, rsel = (lane >> 4) & 1;
+    const int by = blockIdx.y, rbw = (blockIdx.x * 4 + wave) * 2 * RN;  // first 16-row block of this wave
     const int ntg = a.ntg, Mp = a.Mp;
     const size_t items = (size_t)ntg * 16;  // operand items (4 per tile)
-    const uint4* PH = (const uint4*)a.planes;
-    const uint4* PL = PH + items * Mp;
-    const float* PB = (const float*)(PL + items * Mp);
-    const float* PB2 = PB + (size_t)ntg * 4 * Mp;  // the lo plane's biases
+    const int gs0 = blockIdx.z * a.gsteps, gs1 = min(ntg, gs0 + a.gsteps);  // this part's K steps
 
-    // operand chunk c of step g for this lane: 16 hi items, 16 lo items, the
-    // hi biases, the lo biases.  One unconditional load per chunk, the source
-    // picked by selects (a load under a branch makes the compiler wait for it
-    // at once); chunk j of this wave is held in its own register quad (RA).
-    auto src_a = [&](int j, int g) __attribute__((always_inline)) -> const uint4* {
-        const int c = min(wave + 4 * j, GCH - 1);
-        const uint4* ph = PH + (size_t)(16 * g + c) * Mp + GB * by + lane;
-        const uint4* pl = PL + (size_t)(16 * g + c - 16) * Mp + GB * by + lane;
-        const size_t bo = (size_t)(4 * g + (lane >> 4)) * Mp + GB * by + 4 * (lane & 15);
-        const uint4* pb = (const uint4*)((c == 32 ? PB : PB2) + bo);
-        return c < 16 ? ph : c < 32 ? pl : pb;
-    };
-    // chunk j of this wave in buffer buf: the wave-uniform 1 KiB it fills
-    // (lane l's 16 bytes land at + 16 l); the clamped chunk (the lo biases)
-    // is written by every wave with the same data
-    auto dma_a = [&](int j, int g, int buf) __attribute__((always_inline)) {
-        uint4* dst = gemm_at + ((size_t)buf * GCH + min(wave + 4 * j, GCH - 1)) * 64;
-        __builtin_amdgcn_global_load_lds((const void*)src_a(j, g), (__attribute__((address_space(3))) void*)dst, 16,
-                                         0, 0);
-    };
-    // weights of step g for the wave's row blocks (clamped to the last block)
-    auto load_w = [&](uint4* wv, int g) __attribute__((always_inline)) {
+    // the 16-byte words of group g: lane -> weight row (block 2 q + rsel, row
+    // r), k-slots h and 2 + h of its four tiles; blocks past the matrix
+    // repeat the last one
+    const uint4* wp[RN];
+    const uint8_t* sp[RN];
 #pragma unroll
-        for (int q = 0; q < GRB; q++) {
-            const size_t t = (size_t)min(rbw + q, a.nrb - 1) * ntg + g;
-            wv[q] = ((const uint4*)a.w)[t * 64 + lane];
+    for (int q = 0; q < RN; q++) {
+        const size_t t = (size_t)min(rbw + 2 * q + rsel, a.nrb - 1) * ntg;
+        wp[q] = (const uint4*)a.w + t * 64 + 16 * h + r;
+        sp[q] = (const uint8_t*)a.scale + (t * 16 + r) * (TP ? 4 : 8);
+    }
+    auto load_w = [&](uint4 (*wv)[2], uint2* sv, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < RN; q++) {
+            wv[q][0] = wp[q][(size_t)g * 64];
+            wv[q][1] = wp[q][(size_t)g * 64 + 32];
+            if constexpr (TP) sv[q].x = *(const uint32_t*)(sp[q] + (size_t)g * 64);
+            else sv[q] = *(const uint2*)(sp[q] + (size_t)g * 128);
         }
     };
-    // the tile scales of step g for the wave's rows into its 1 KiB of the
-    // scale area (buffer buf) by one direct load: q4t 16 B per lane = two
-    // rows' four f16 scales, lane l -> row block l / 8, rows 2 (l % 8) ..;
-    // q4tp 4 B per lane = one row's four rung codes, lane l -> row block
-    // l / 16, row l % 16 (lanes past the wave's rows repeat the last block)
-    uint8_t* sarea = (uint8_t*)(gemm_at + (size_t)2 * GCH * 64);
-    auto dma_s = [&](int g, int buf) __attribute__((always_inline)) {
-        uint8_t* dst = sarea + (size_t)(buf * 4 + wave) * 1024;
-        if constexpr (TP) {
-            const int q = min(lane >> 4, GRB - 1);
-            const size_t t = (size_t)min(rbw + q, a.nrb - 1) * ntg + g;
-            __builtin_amdgcn_global_load_lds((const void*)((const uint32_t*)a.scale + t * 16 + (lane & 15)),
-                                             (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
-        } else {
-            const int q = min(lane >> 3, GRB - 1);
-            const size_t t = (size_t)min(rbw + q, a.nrb - 1) * ntg + g;
-            __builtin_amdgcn_global_load_lds((const void*)((const uint2*)a.scale + t * 16 + 2 * (lane & 7)),
-                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    // the operand of stage i (of the whole K: tiles TPS i ..) into ring slot
+    // buf: chunk c = plane, item, 64 rows
+    auto dma = [&](int i, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NCH; j++) {
+            const int c = wave * NCH + j;
+            const int rh = c % (BM / 64), it = (c / (BM / 64)) % (4 * TPS), pl = c / (4 * TPS * (BM / 64));
+            const uint4* src = (const uint4*)a.planes +
+                               ((size_t)pl * items + 4 * TPS * i + it) * Mp + BM * by + 64 * rh + lane;
+            uint4* dst = gemm_at + ((size_t)buf * 8 * TPS + pl * 4 * TPS + it) * BM + 64 * rh;
+            __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
         }
     };
+    const int i0 = gs0 * SPG, i1 = gs1 * SPG;  // stages
+    uint4 wv[RN][2];
+    uint2 sv[RN];
+#pragma unroll
+    for (int k = 0; k < NB - 1; k++) dma(min(i0 + k, i1 - 1), (i0 + k) % NB);
+    load_w(wv, sv, gs0);
     if constexpr (TP) {  // 32-rung ladders of the wave's rows (quant.rs:399-410)
 #pragma unroll
-        for (int q = 0; q < GRB; q++) {
-            if (s == 0) {
-                const float2 p = a.rowp[min(rbw + q, a.nrb - 1) * 16 + r];
+        for (int q = 0; q < RN; q++) {
+            if (h == 0) {
+                const float2 p = a.rowp[min(rbw + 2 * q + rsel, a.nrb - 1) * 16 + r];
+                float* row = lad + ((wave * RN + q) * 32 + c32) * 32;
                 float tv = p.x;
-                lad[wave][(q * 16 + r) * 33] = tv;
+                row[c32] = tv;
                 for (int c = 1; c < 32; c++) {
                     tv = tv * p.y;
-                    lad[wave][(q * 16 + r) * 33 + c] = tv;
+                    row[c ^ c32] = tv;
                 }
             }
         }
     }
-    float4v acc[GRB][4];
+    float16v acc[RN][MB];
 #pragma unroll
-    for (int q = 0; q < GRB; q++)
+    for (int q = 0; q < RN; q++)
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) acc[q][mb] = float4v{0.f, 0.f, 0.f, 0.f};
-
-    const int gs0 = blockIdx.z * a.gsteps, gs1 = min(ntg, gs0 + a.gsteps);  // this part's K steps
-    uint4 wA[GRB], wB[GRB];
-#pragma unroll
-    for (int j = 0; j < GJ; j++) dma_a(j, gs0, 0);
-    dma_s(gs0, 0);
-    load_w(wA, gs0);
+        for (int mb = 0; mb < MB; mb++) acc[q][mb] = float16v{};
     wait_vmcnt<0>();
     __syncthreads();
 
-    auto compute = [&](int buf, const uint4* wv) __attribute__((always_inline)) {
-        const uint4* A = gemm_at + (size_t)buf * GCH * 64;
-        // this step's scale words of the lane's rows in LDS (q4t: [q][r] four
-        // f16; q4tp: [q][r] u32 of four 5-bit codes), read per tile
-        const uint8_t* sb = sarea + (size_t)(buf * 4 + wave) * 1024;
-        const float4v* Bias = (const float4v*)(A + 32 * 64);   // hi plane's [tile][64 rows] f32
-        const float4v* BiasL = (const float4v*)(A + 33 * 64);  // lo plane's
-#pragma unroll 1
-        for (int t = 0; t < 4; t++) {
-            half8 bq[GRB];
-            float sc[GRB];
-#pragma unroll
-            for (int q = 0; q < GRB; q++) {
-                const uint32_t wd = t == 0 ? wv[q].x : t == 1 ? wv[q].y : t == 2 ? wv[q].z : wv[q].w;
-                bq[q] = dq_nib_word(wd);
-                if constexpr (TP) {
-                    const uint32_t code = ((const uint32_t*)sb)[q * 16 + r];
-                    sc[q] = lad[wave][(q * 16 + r) * 33 + ((code >> (5 * t)) & 31)];
-                } else {
-                    sc[q] = f16_bits_to_f32(((const uint16_t*)sb)[(q * 16 + r) * 4 + t]);
-                }
-            }
-#pragma unroll
-            for (int mb = 0; mb < 4; mb++) {
-                const half8 xh = __builtin_bit_cast(half8, A[(4 * t + s) * 64 + 16 * mb + r]);
-                const half8 xl = __builtin_bit_cast(half8, A[(16 + 4 * t + s) * 64 + 16 * mb + r]);
-                const float4v cb = Bias[t * 16 + 4 * mb + s];  // rows 16 mb + 4 s .. + 3
-                const float4v cbl = BiasL[t * 16 + 4 * mb + s];
-#pragma unroll
-                for (int q = 0; q < GRB; q++) {
-                    // hi and lo in accumulators of their own: each tile sum is
-                    // exact only within one plane
-                    float4v d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, bq[q], cb, 0, 0, 0);
-                    d += __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, bq[q], cbl, 0, 0, 0);
-                    acc[q][mb] += d * sc[q];
-                }
-            }
-        }
+    // tile tt of a group (its words and scales in registers): the weights of
+    // 32-row block q, k half j, and its scale
+    auto wword = [&](const uint4& w4, int tt) __attribute__((always_inline)) -> uint32_t {
+        return tt == 0 ? w4.x : tt == 1 ? w4.y : tt == 2 ? w4.z : w4.w;
     };
-
-    // The next step's operand and tile scales (into the other buffer,
-    // directly) and weights go out before this step's MFMAs; the wait covers
-    // the direct loads only (the GRB weight loads after them stay in flight), and the barrier
-    // lets every wave's chunks land before they are read and keeps the
-    // buffer being read from being refilled.  Past the last step the loads
-    // repeat it into the buffer no one reads.
-    for (int g = gs0; g < gs1; g += 2) {
-        {
-            const int g_ = min(g + 1, gs1 - 1);
-#pragma unroll
-            for (int j = 0; j < GJ; j++) dma_a(j, g_, 1);
-            dma_s(g_, 1);
-            load_w(wB, g_);
-            compute(0, wA);
-            wait_vmcnt<GRB>();
+    auto tscale = [&](const uint2& s2, int tt, int q) __attribute__((always_inline)) -> float {
+        float f;
+        if constexpr (TP) {
+            f = lad[((wave * RN + q) * 32 + c32) * 32 + (((s2.x >> (5 * tt)) & 31) ^ c32)];
+        } else {
+            const uint32_t u = tt < 2 ? s2.x : s2.y;
+            f = f16_bits_to_f32((tt & 1) == 0 ? u & 0xffffu : u >> 16);
         }
-        lds_sync();
-        if (g + 1 >= gs1) break;
-        {
-            const int g_ = min(g + 2, gs1 - 1);
+        asm("" : "+v"(f));  // (an f32 register: plain FMAs)
+        return f;
+    };
+    half8 bw[2][RN][2];
+    float sc[2][RN];
 #pragma unroll
-            for (int j = 0; j < GJ; j++) dma_a(j, g_, 0);
-            dma_s(g_, 0);
-            load_w(wA, g_);
-            compute(1, wB);
-            wait_vmcnt<GRB>();
-        }
-        lds_sync();
+    for (int q = 0; q < RN; q++) {
+        sc[0][q] = tscale(sv[q], 0, q);
+#pragma unroll
+        for (int j = 0; j < 2; j++) bw[0][q][j] = dq_signed(wword(wv[q][j], 0));
     }
 #pragma unroll
-    for (int q = 0; q < GRB; q++) {
-        const int n = (rbw + q) * 16 + r;
-        if (rbw + q >= a.nrb || n >= a.N) continue;
+    for (int q = 0; q < RN; q++) sc[1][q] = 0.f;
+    float16v d[2] = {};
+    // Stage i: the operand of stage i + NB - 1 goes out (into the slot that
+    // stage i - 1 has left), in a group's first stage also the next group's
+    // weights, then stage i's MFMAs; the wait covers stage i + 1's operand
+    // and leaves the loads issued after it in flight.  Past the last stage
+    // the loads repeat it into slots no one reads.
+    // The outputs go in blocks of 32 x 32; a block's four MFMAs (lo then hi,
+    // one accumulator) run while the block before it is scaled into its f32
+    // sums, the next operand rows are read and the next tile's weights
+    // unpacked, some of that beside each MFMA (the scheduling barriers keep
+    // the compiler from moving it in front of them).
+    constexpr int NBLK = TPS * MB * RN;
+    for (int g = gs0; g < gs1; g++) {
+        uint4 wn[RN][2];
+        uint2 sn[RN];
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+        for (int st = 0; st < SPG; st++) {
+            const int i = g * SPG + st;
+            const uint4* A = gemm_at + (size_t)(i % NB) * 8 * TPS * BM + h * BM + c32;
+            // operand fragment k (lo0, lo1, hi0, hi1) of rows mb, tile t
+            auto frag = [&](int t, int mb, int k) __attribute__((always_inline)) {
+                return __builtin_bit_cast(half8, A[(4 * t + 2 * (k & 1) + (k < 2 ? 4 * TPS : 0)) * BM + 32 * mb]);
+            };
+            half8 xa[2][4];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int b = GB * by + 16 * mb + 4 * s + v;
+            for (int k = 0; k < 4; k++) xa[0][k] = frag(0, 0, k);
+            dma(min(i + NB - 1, i1 - 1), (i + NB - 1) % NB);
+            // (the wait below counts the weights as issued after the operand)
+            __builtin_amdgcn_sched_barrier(0);
+            if (st == 0) load_w(wn, sn, min(g + 1, gs1 - 1));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int n = 0; n < NBLK; n++) {
+                const int q = n % RN, mb = (n / RN) % MB, t = n / (RN * MB), tt = TPS * st + t;
+                // the block before (n = 0: the last of the stage before)
+                const int np = n + NBLK - 1, pq = np % RN, pm = (np / RN) % MB, pt = tt - (n % (RN * MB) == 0);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    d[n & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                        xa[(n / RN) & 1][k], bw[tt & 1][q][k & 1], k == 0 ? float16v{} : d[n & 1], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    // the next rows' fragments, during the last block of these
+                    const int e = n / RN + 1;
+                    if (q == RN - 1 && e < TPS * MB) xa[e & 1][k] = frag(e / MB, e % MB, k);
+                    // the next tile's weight words, one per block, then its scales
+                    const int bi = n % (RN * MB), sq = bi - RN * MB + RN;
+                    if (k == 0 && bi < 2 * RN)
+                        bw[(tt + 1) & 1][bi / 2][bi & 1] =
+                            dq_signed(tt < 3 ? wword(wv[bi / 2][bi & 1], tt + 1) : wword(wn[bi / 2][bi & 1], 0));
+                    if (k == 3 && sq >= 0)
+                        sc[(tt + 1) & 1][sq] = tt < 3 ? tscale(sv[sq], tt + 1, sq) : tscale(sn[sq], 0, sq);
+                    if (k > 0) {
+                        const int v0 = k == 1 ? 0 : k == 2 ? 5 : 10, v1 = k == 1 ? 5 : k == 2 ? 10 : 16;
+#pragma unroll
+                        for (int v = 0; v < 16; v++)
+                            if (v >= v0 && v < v1)
+                                acc[pq][pm][v] = fmaf(d[np & 1][v], sc[pt & 1][pq], acc[pq][pm][v]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // loads issued after stage i + 1's operand: the NB - 2 stages
+            // after it and one group's weights
+            wait_vmcnt<(NB - 2) * NCH + NW>();
+            lds_sync();
+        }
+#pragma unroll
+        for (int q = 0; q < RN; q++) {
+            wv[q][0] = wn[q][0];
+            wv[q][1] = wn[q][1];
+            sv[q] = sn[q];
+        }
+    }
+    wait_vmcnt<0>();  // (no load into this workgroup's LDS outlives it)
+#pragma unroll
+    for (int v = 0; v < 16; v++)  // the last block (tile 3 of a group)
+        acc[RN - 1][MB - 1][v] = fmaf(d[(NBLK - 1) & 1][v], sc[1][RN - 1], acc[RN - 1][MB - 1][v]);
+#pragma unroll
+    for (int q = 0; q < RN; q++) {
+        const int n = (rbw + 2 * q) * 16 + c32;
+        if (n >= a.N) continue;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int b = BM * by + 32 * mb + 8 * (v >> 2) + 4 * h + (v & 3);
                 if (b < a.M) {
-                    const float val = acc[q][mb][v] * a.xs[b] * 16777216.0f;
+                    const float val = acc[q][mb][v] * a.xs[b];
                     if (a.part) {
                         a.part[((size_t)blockIdx.z * a.M + b) * a.N + n] = val;
                     } else {
@@ -394,11 +446,10 @@ static thread_local size_t g_gemm_part_cap = 0;
 
 // K parts for a grid of base workgroups over nsteps K steps: doubled while
 // the grid is below one workgroup per CU (256), at least 4 steps a part.
-// Measured on MI355X: at m = 256 (prefill chunks) the down projection
-// 1024x3072 (64 workgroups unsplit) and wo 1024x2048 take 4 parts; q4t
-// 12288x4096 at m = 64 (192 workgroups) 2 parts, 71 -> 56 us; qkv at
-// m = 256 (256 workgroups) split in 2 made the prefill slower (32.9 ->
-// 33.6 ms).
+// Measured on MI355X: q4t 1024x3072 m = 2048 (128 workgroups unsplit) 77 us
+// in one part, 68 in two, 74 in four; q4tp 2048x6144 m = 200 (64) 90 / 61 /
+// 46 us in 1 / 2 / 4; q4t 12288x4096 m = 64 (96) 62 / 46 / 42; a grid of
+// 256 or more loses (2048x6144 m = 2048 161 -> 162, 6144x1024 88 -> 125).
 static int gemm_kparts(long base, int nsteps) {
     static const int env = [] {
         const char* e = getenv("CMF_GEMM_SPLITK");
@@ -412,9 +463,8 @@ static int gemm_kparts(long base, int nsteps) {
 
 size_t gemm_planes_bytes(const DevWeight& w, int mp) {
     // q8: three planes of nk * 64 * Mp B; q4: hi + lo 2 * items * Mp * 16 B
-    // and the two tables of tile biases 2 * tiles * Mp * 4 B
     if (w.dtype == DT_Q8ROW) return (size_t)w.kchunks * 64 * mp * 3;
-    return (size_t)w.kchunks * 16 * mp * 32 + (size_t)w.kchunks * 4 * mp * 8;
+    return (size_t)w.kchunks * 16 * mp * 32;
 }
 
 int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st) {
@@ -490,21 +540,18 @@ int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool res
         else hipLaunchKernelGGL((k_gemm_q8<1>), grid, dim3(256), GEMM_Q8_AT_BYTES, st, a);
         return reduce(nz);
     }
-    // four row blocks per wave once that still leaves ~4 workgroups per CU
-    const bool big = (long)((a.nrb + 15) / 16) * (mp / GB) >= 1024;
-    // two row blocks per wave (half the operand re-reads) while that still
-    // gives >= 384 workgroups: measured 12288x4096 m=256 160 -> 126 us, but
-    // 6144x1024 m=256 (192 workgroups) 30.7 -> 38.8 us
-    const int grb_small = !big && (long)((a.nrb + 7) / 8) * (mp / GB) >= 384 ? 2 : 1;
-    const int rbwg = big ? 16 : 4 * grb_small;
+    // 64 rows a wave (half the operand reads of 32) while that gives a
+    // workgroup to at least half the CUs, else 32: q4t 12288x4096 m = 2048
+    // 412 us at 64, 457 at 32; q4tp 6144x2048 m = 200 (96 workgroups) 50 and
+    // 40, 1000x1056 m = 77 25 and 19
+    const int rn = (long)((a.nrb + 15) / 16) * (mp / GB) >= 128 ? 2 : 1;
+    const int rbwg = 8 * rn;
     const int gx = (a.nrb + rbwg - 1) / rbwg, nz = split((long)gx * (mp / GB), a.ntg);
     if (nz < 0) return fail("gemm: split-K buffer");
     const dim3 grid(gx, mp / GB, nz);
-    const void* kf = w.dtype == DT_Q4T
-                         ? (big ? (const void*)k_gemm_q4<DT_Q4T, 4>
-                                : (grb_small == 2 ? (const void*)k_gemm_q4<DT_Q4T, 2> : (const void*)k_gemm_q4<DT_Q4T, 1>))
-                         : (big ? (const void*)k_gemm_q4<DT_Q4TP, 4>
-                                : (grb_small == 2 ? (const void*)k_gemm_q4<DT_Q4TP, 2> : (const void*)k_gemm_q4<DT_Q4TP, 1>));
+    const bool q4t = w.dtype == DT_Q4T;
+    const void* kf = rn == 2 ? (q4t ? (const void*)k_gemm_q4<DT_Q4T, 2> : (const void*)k_gemm_q4<DT_Q4TP, 2>)
+                             : (q4t ? (const void*)k_gemm_q4<DT_Q4T, 1> : (const void*)k_gemm_q4<DT_Q4TP, 1>);
     {
         // the operand tile's dynamic LDS is above the default 64 KiB limit
         static std::mutex mu;

@@ -251,8 +251,8 @@ constexpr float Q4_BIAS = -4.76837158203125e-07f;  // -8 * 2^-24: the format's n
 // tile (T2 right after T1), zero for rows in [M, bstride).  With bstride ==
 // 16 and M <= 8 (the GEMVs whose A rows 8 + b carry the lo plane of batch
 // row b) T1[t][8 + b] holds the lo bias as well.  M is the planes' row
-// stride (the batch of a GEMV; the padded row count of a GEMM, with bstride
-// = M).  The q4 kernels multiply by the nibbles as f16 denormals n * 2^-24
+// stride (the batch of a GEMV; the padded row count of a GEMM, which takes
+// no biases: bstride = 0).  The q4 kernels multiply by the nibbles as f16 denormals n * 2^-24
 // and start each tile's accumulator at the bias of its plane, so that
 // D = 2^-24 * sum((n - 8) * x) / xs exactly.  nthr must be a multiple of 64:
 // the four items of a tile sit in lanes 4t..4t+3 of one wave, which add
@@ -307,7 +307,7 @@ __device__ inline void prep16_row(const float* x, int K, float amax, int ntiles,
                                          hv[4] | (hv[5] << 16), hv[6] | (hv[7] << 16));
         *(uint4*)(pl + off) = make_uint4(lv[0] | (lv[1] << 16), lv[2] | (lv[3] << 16),
                                          lv[4] | (lv[5] << 16), lv[6] | (lv[7] << 16));
-        if (s == 0) q4_put_bias(bias, ntiles, bstride, M, t, b, sh, sl);
+        if (s == 0 && bstride) q4_put_bias(bias, ntiles, bstride, M, t, b, sh, sl);
     }
 }
 

@@ -115,10 +115,10 @@ __device__ inline void prep_src_row(XSrc s, int K, int fmt, int nk, uint8_t* __r
     am = 0.f;
     for (int q = 0; q < nw; q++) am = fmaxf(am, redm[q]);
     // row stride of the planes: the batch (GEMV operands) or a padded row
-    // count (GEMM operands, whose tile biases share that stride)
+    // count (GEMM operands, without tile biases)
     const int ms = mstride ? mstride : m;
     if (fmt == DT_Q8ROW) prep8_row(vals, K, am, nk, b, ms, planes, xs, tid, nt);
-    else prep16_row(vals, K, am, nk, b, ms, planes, xs, tid, nt, mstride ? mstride : 16);
+    else prep16_row(vals, K, am, nk, b, ms, planes, xs, tid, nt, mstride ? 0 : 16);
 }
 
 }  // namespace cmf
