@@ -42,6 +42,152 @@ __global__ __launch_bounds__(512) void k_prep_src(XSrc s, int K, int fmt, int nk
     prep_src_row(s, K, fmt, nk, planes, xs, mstride, b, mstride ? m : gridDim.x, vals);
 }
 
+// ---------------------------------------------------------------------------
+// GEMM operand of many rows: one wave per row, the row in its registers (NI
+// items of 8 (q4) or 16 (q8) columns per lane), so that a row costs one
+// memory round trip, two wave reductions (f64 sum of squares, max|x|) and
+// its stores, with no LDS and no barrier.  The eight waves of a workgroup
+// take eight consecutive rows: their 16-byte items make whole 128-byte lines
+// of the row-interleaved planes, merged in one L2.  Bound by memory latency
+// and the stores.  Producers: XS_ROWS, XS_NORM, XS_SILU, XS_SILU8 (the
+// values of prep_src_row; its f64 sums in another order).  grid (m / 8),
+// 512.
+// ---------------------------------------------------------------------------
+template <bool Q8, int MODE, int NI>
+__global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, uint8_t* __restrict__ planes,
+                                                   float* __restrict__ xs, int Mp, int m) {
+    constexpr int C = Q8 ? 16 : 8;
+    const int lane = threadIdx.x & 63, b = blockIdx.x * 8 + (threadIdx.x >> 6);
+    if (b >= m) return;
+    const float* row = s.x + (size_t)b * s.ldx;
+    float v[NI][C];
+    float4 wv[MODE == XS_NORM ? NI : 1][C / 4];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int c0 = (lane + 64 * i) * C;
+        const bool in = c0 < K;  // (K % C == 0: an item is all inside or all past the row)
+        const int c = in ? c0 : 0;
+#pragma unroll
+        for (int q = 0; q < C / 4; q++) {
+            float4 x;
+            if constexpr (MODE == XS_SILU || MODE == XS_SILU8) {
+                // gate and up of columns c + 4 q ..: [0, K) / [K, 2 K), or
+                // interleaved 8 / 8
+                const float* gp = MODE == XS_SILU ? row + c + 4 * q : row + 2 * c + 16 * (q >> 1) + 4 * (q & 1);
+                const float4 g = *(const float4*)gp, u = *(const float4*)(gp + (MODE == XS_SILU ? s.K : 8));
+                x.x = (g.x / (1.0f + expf(-g.x))) * u.x;
+                x.y = (g.y / (1.0f + expf(-g.y))) * u.y;
+                x.z = (g.z / (1.0f + expf(-g.z))) * u.z;
+                x.w = (g.w / (1.0f + expf(-g.w))) * u.w;
+            } else {
+                x = *(const float4*)(row + c + 4 * q);
+            }
+            if constexpr (MODE == XS_NORM) wv[i][q] = *(const float4*)(s.w + c + 4 * q);
+            v[i][4 * q] = in ? x.x : 0.f;
+            v[i][4 * q + 1] = in ? x.y : 0.f;
+            v[i][4 * q + 2] = in ? x.z : 0.f;
+            v[i][4 * q + 3] = in ? x.w : 0.f;
+        }
+    }
+    if constexpr (MODE == XS_NORM) {
+        double ss = 0.0;
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int j = 0; j < C; j++) ss += (double)v[i][j] * (double)v[i][j];
+        ss = wave_sum(ss);
+        const float inv = 1.0f / (float)sqrt(ss / (double)K + s.eps);
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int j = 0; j < C; j++) {
+                const float4 w4 = wv[i][j >> 2];
+                v[i][j] = v[i][j] * inv * ((j & 3) == 0 ? w4.x : (j & 3) == 1 ? w4.y : (j & 3) == 2 ? w4.z : w4.w);
+            }
+    }
+    float am = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int j = 0; j < C; j++) am = fmaxf(am, fabsf(v[i][j]));
+    am = wave_max(am);
+    const size_t plane = (size_t)nitems * Mp * 16;
+    if constexpr (Q8) {
+        const float sx = am > 0.f ? am / 127.0f : 1.0f;
+        const float inv = 1.0f / sx;
+        if (lane == 0) xs[b] = sx;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int idx = lane + 64 * i;
+            if (idx >= nitems) continue;
+            uint32_t w0[4] = {}, w1[4] = {}, w2[4] = {};
+#pragma unroll
+            for (int j = 0; j < 16; j++) q8_split(v[i][j] * inv, j & 3, w0[j >> 2], w1[j >> 2], w2[j >> 2]);
+            uint8_t* p = planes + ((size_t)idx * Mp + b) * 16;
+            *(uint4*)p = make_uint4(w0[0], w0[1], w0[2], w0[3]);
+            *(uint4*)(p + plane) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
+            *(uint4*)(p + 2 * plane) = make_uint4(w2[0], w2[1], w2[2], w2[3]);
+        }
+    } else {
+        float scale, xsv;
+        q4_fix_scale(am, scale, xsv);
+        if (lane == 0) xs[b] = xsv;
+        constexpr int ord[8] = {0, 4, 2, 6, 1, 5, 3, 7};
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int idx = lane + 64 * i;
+            if (idx >= nitems) continue;
+            uint32_t hv[4] = {}, lv[4] = {};
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                _Float16 h, l;
+                q4_fix_split(v[i][ord[j]] * scale, h, l);
+                hv[j >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, h) << (16 * (j & 1));
+                lv[j >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, l) << (16 * (j & 1));
+            }
+            uint8_t* p = planes + ((size_t)idx * Mp + b) * 16;
+            *(uint4*)p = make_uint4(hv[0], hv[1], hv[2], hv[3]);
+            *(uint4*)(p + plane) = make_uint4(lv[0], lv[1], lv[2], lv[3]);
+        }
+    }
+}
+
+// The instance that holds nitems per row (nullptr: none; the row's columns
+// per lane: up to 128)
+typedef void (*PrepGemm)(XSrc, int, int, uint8_t*, float*, int, int);
+template <bool Q8, int MODE>
+static PrepGemm prep_gemm_pick(int nitems) {
+    constexpr int D = Q8 ? 2 : 1;
+    const int ni = (nitems + 63) / 64 * D;
+    if (ni <= 2) return k_prep_gemm<Q8, MODE, 2 / D>;
+    if (ni <= 4) return k_prep_gemm<Q8, MODE, 4 / D>;
+    if (ni <= 6) return k_prep_gemm<Q8, MODE, 6 / D>;
+    if (ni <= 8) return k_prep_gemm<Q8, MODE, 8 / D>;
+    if constexpr (MODE != XS_NORM) {  // (a norm's weights would spill past 64 columns per lane)
+        if (ni <= 12) return k_prep_gemm<Q8, MODE, 12 / D>;
+        if (ni <= 16) return k_prep_gemm<Q8, MODE, 16 / D>;
+    }
+    return nullptr;
+}
+static PrepGemm prep_gemm_kernel(const DevWeight& w, const XSrc& s, int K) {
+    const bool q8 = w.dtype == DT_Q8ROW;
+    // whole items and 16-byte loads
+    if (K % (q8 ? 16 : 8) || s.ldx % 4 || (uintptr_t)s.x % 16) return nullptr;
+    const int nitems = w.kchunks * (q8 ? 4 : 16);
+    switch (s.mode) {
+        case XS_ROWS: return q8 ? prep_gemm_pick<true, XS_ROWS>(nitems) : prep_gemm_pick<false, XS_ROWS>(nitems);
+        case XS_NORM:
+            if ((uintptr_t)s.w % 16) return nullptr;
+            return q8 ? prep_gemm_pick<true, XS_NORM>(nitems) : prep_gemm_pick<false, XS_NORM>(nitems);
+        case XS_SILU:
+            if (s.K % 4) return nullptr;
+            return q8 ? prep_gemm_pick<true, XS_SILU>(nitems) : prep_gemm_pick<false, XS_SILU>(nitems);
+        case XS_SILU8:
+            return q8 ? prep_gemm_pick<true, XS_SILU8>(nitems) : prep_gemm_pick<false, XS_SILU8>(nitems);
+        default: return nullptr;
+    }
+}
+
 // The a8w8 operand (split_act, qtensor.rs:9237-9281) of row b of x: rms =
 // sqrt(sum(x*x) / n) (f32 products, f64 sum), outliers |x| > 8 rms listed
 // exactly in index order (idx/val, count), sx = max|x| of the rest / 127
@@ -198,6 +344,10 @@ int launch_prep_src_gemm(const DevWeight& w, const XSrc& src, int m, int mstride
     if (K < 1 || K > w.cols || K > 16384) return fail("prep: operand length must be 1..min(cols, 16384)");
     if (src.mode == XS_CAT && (src.H < 1 || src.H >= K)) return fail("prep: bad concat split");
     const int nk = w.dtype == DT_Q8ROW ? w.kchunks : w.kchunks * 4;
+    if (PrepGemm pk = prep_gemm_kernel(w, src, K)) {
+        hipLaunchKernelGGL(pk, dim3((m + 7) / 8), dim3(512), 0, st, src, K, nk * 4, planes, xs, mstride, m);
+        return CMF_OK;
+    }
     // (256 threads a row: all of a 2048-row chunk's workgroups resident at
     // once; measured on MI355X, the 2048-position prefill 12.45 -> 12.21 ms
     // against 512, 12.5 ms at 128)
