@@ -499,6 +499,9 @@ bool gemv_fuse_pays(const DevWeight& w, int m) {
 static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int grid_override, int gridy,
                        hipStream_t st) {
     const int m = a.m;
+    // (a job list of one is still a job list: the ungrouped kernels would
+    // read the prototype's weight instead of the job's expert)
+    const bool grouped = a.jobs != nullptr;
     if (a.src.K == 0) a.src.K = w.cols;
     // K steps of 1 KiB per row block: q8 chunks of 64 columns, q4 groups of
     // 4 tiles (128 columns)
@@ -514,7 +517,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     if (a.src.mode == XS_GLOBAL && a.src.cs) {
         // chunk-scaled q8 planes: the planes (1 KiB aligned) then the chunk
         // scales, rounded to whole 1 KiB direct-load chunks
-        if (w.dtype != DT_Q8ROW || a.src.cs_ld != w.kchunks || gridy > 1)
+        if (w.dtype != DT_Q8ROW || a.src.cs_ld != w.kchunks || grouped)
             return fail("gemv: chunk-scaled operands are q8, contiguous, ungrouped");
         lds = ((lds_bytes(w, m) + 1023) & ~(size_t)1023) + (((size_t)m * w.kchunks * 4 + 1023) & ~(size_t)1023);
         if (lds > LDSX_MAX) return fail("gemv: chunk-scaled operand too large for LDS");
@@ -525,14 +528,14 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
         xm = lds ? XM_PREP : XM_GLOBAL;
     } else {
         lds = fused_lds_bytes(w, a.src, m);
-        if (!lds || gridy > 1) return fail("gemv: this operand must be prepared (launch_prep_src)");
+        if (!lds || grouped) return fail("gemv: this operand must be prepared (launch_prep_src)");
         xm = XM_FUSED;
     }
     // M = 1 over a prepared operand: the per-wave operand-slice kernels
     // (k_gemv_q8_m1, k_gemv_q4t_m1), one workgroup per row block
     // (CMF_GEMV_M1=0 keeps the general kernel)
     static const int m1_env = env_int("CMF_GEMV_M1", 1);
-    if (m1_env && m == 1 && xm == XM_PREP && gridy == 1 && grid_override <= 0 && ks_override <= 0 &&
+    if (m1_env && m == 1 && xm == XM_PREP && !grouped && grid_override <= 0 && ks_override <= 0 &&
         a.epi == EPI_NONE && (w.dtype == DT_Q8ROW || w.dtype == DT_Q4T)) {
         int ks1 = 0;
         size_t l1 = 0;
@@ -548,7 +551,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     // q4t M = 1 from the f32 row (XS_ROWS): the kernel that stages its own
     // operand slices (CMF_GEMV_M1X=0 keeps the general fused kernel)
     static const int m1x_env = env_int("CMF_GEMV_M1X", 1);
-    if (m1x_env && m == 1 && xm == XM_FUSED && a.src.mode == XS_ROWS && w.dtype == DT_Q4T && gridy == 1 &&
+    if (m1x_env && m == 1 && xm == XM_FUSED && a.src.mode == XS_ROWS && w.dtype == DT_Q4T && !grouped &&
         grid_override <= 0 && ks_override <= 0 && a.epi == EPI_NONE && a.src.K % 8 == 0) {
         int ks1 = 0;
         GemvKernel k1 = q4t_kernel_m1x(w.kchunks, a.resid, &ks1);
@@ -573,7 +576,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     //    q4tp at m > 1 keeps the 16 x 4 kernel, whose in-place variant
     //    would spill).
     static const int g_env = env_int("CMF_GEMV_G", -1), s6_env = env_int("CMF_GEMV_S6", -1);
-    const bool alt_ok = w.dtype != DT_Q8ROW && gridy == 1 && grid_override <= 0 && ks_override <= 0 &&
+    const bool alt_ok = w.dtype != DT_Q8ROW && !grouped && grid_override <= 0 && ks_override <= 0 &&
                         a.src.mode == XS_GLOBAL && !a.src.cs;
     const bool g3 = alt_ok && w.kchunks <= 32 && a.nrb >= 3 * num_cus() &&
                     (g_env == 3 || (g_env < 0 && m >= 4 && m <= 8));
@@ -634,7 +637,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     // 12288x4096 m = 16 20.0 -> 13.0 us at RB = 3; 4096x12288, 256 row
     // blocks, 19.8 -> 25.9 us, so not there)
     const bool share_rb = xm == XM_GLOBAL && m > 8;
-    if (gridy == 1 && grid_override <= 0 && pick(2)) {
+    if (!grouped && grid_override <= 0 && pick(2)) {
         for (int c = 2; c <= 3; c++) {
             const bool want = rb_env > 0 ? c == rb_env
                               : share_rb ? a.nrb >= c * num_cus()
@@ -652,7 +655,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     // operand copy; measured on MI355X for the config-5 layer 56.6 -> 53.0 us
     // (3: 54.8 us).  CMF_GEMV_GRB overrides.
     static const int grb_env = env_int("CMF_GEMV_GRB", 2);
-    if (gridy > 1 && grb_env > 1 && pick(grb_env)) {
+    if (grouped && grb_env > 1 && pick(grb_env)) {
         GemvKernel kc = pick(grb_env);
         const int oc = resident_per_cu(kc, threads, lds);
         if (oc >= 1) {
@@ -664,7 +667,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
     // one workgroup per RB row blocks while the CUs hold them all at once;
     // grouped launches always give every job its full set
     const int units = (a.nrb + rb - 1) / rb;
-    int grid = gridy > 1 ? units : std::min(units, occ * num_cus());
+    int grid = grouped ? units : std::min(units, occ * num_cus());
     if (grid_override > 0) grid = std::min(grid_override, a.nrb);
     void* args[] = {&a};
     CMF_HIP(hipLaunchKernel((const void*)k, dim3(grid, gridy), dim3(threads), args, lds, st));
