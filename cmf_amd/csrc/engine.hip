@@ -58,19 +58,46 @@ __global__ __launch_bounds__(256) void k_rms_rows(const float* __restrict__ x, i
 }
 
 // Router logits of a dense f32 router (QTensor::F32 matvec, pool.rs:535-548):
-// logits[b][e] = sum_k W[e][k] x[b][k], one wave per expert row, the rows of
-// x from L2.
-__global__ __launch_bounds__(256) void k_router_f32(const float* __restrict__ W, const float* __restrict__ x,
-                                                    int ne, int H, int nb, float* __restrict__ out) {
-    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (e >= ne) return;  // uniform over the wave
-    const float* wr = W + (size_t)e * H;
-    for (int b = 0; b < nb; b++) {
-        const float* xr = x + (size_t)b * H;
-        float acc = 0.f;
-        for (int k = lane; k < H; k += 64) acc += wr[k] * xr[k];
-        acc = wave_sum(acc);
-        if (lane == 0) out[(size_t)b * ne + e] = acc;
+// out[b][e] = sum_k W[e][k] x[b][k] on the f32 MFMA 16x16x4: a workgroup
+// owns 16 rows x 16 experts, its 16 waves take the 16-column pieces of K in
+// turn and meet in LDS in wave order.  Lane (r, s) loads columns 4 s .. of a
+// piece of row r of x and of W, and the four MFMAs of a piece take one of
+// the four each (the same column permutation on both sides).  Bound by
+// latency: at one tile the loads of a wave are all in flight.  Measured on
+// MI355X, 128 experts x 2048: 16 rows 127 us with a wave per expert that
+// walked the rows one after another.  grid (experts / 16, rows / 16), 1024.
+__global__ __launch_bounds__(1024) void k_router_f32(const float* __restrict__ W, const float* __restrict__ x,
+                                                     int ne, int H, int nb, float* __restrict__ out) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ f4 part[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, s = lane >> 4;
+    const int e0 = blockIdx.x * 16, b0 = blockIdx.y * 16;
+    const float* xr = x + (size_t)min(b0 + r, nb - 1) * H + 4 * s;
+    const float* wr = W + (size_t)min(e0 + r, ne - 1) * H + 4 * s;
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 16 * wave; c0 < H; c0 += 1024) {  // four pieces at a time (H % 32 == 0)
+        f4 a[4], w[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int c = c0 + 256 * u, ca = c < H ? c : c0;
+            a[u] = *(const f4*)(xr + ca);
+            w[u] = *(const f4*)(wr + ca);
+            if (c >= H) a[u] = w[u] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j], w[u][j], acc, 0, 0, 0);
+    }
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    f4 t = part[0][lane];
+    for (int q = 1; q < 16; q++) t += part[q][lane];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int b = b0 + 4 * s + v, e = e0 + r;
+        if (b < nb && e < ne) out[(size_t)b * ne + e] = t[v];
     }
 }
 
@@ -114,6 +141,10 @@ struct cmf_model_s {
     // prefill chunk buffers [prefill_chunk() rows] (allocated by the first prefill)
     float *pf_h = nullptr, *pf_qkv = nullptr, *pf_ao = nullptr, *pf_gu = nullptr, *pf_hm = nullptr, *pf_q = nullptr;
     int* pf_toks = nullptr;
+    void* pf_moe = nullptr;  // routed-expert blocks: moe_prefill_scratch bytes, router logits [chunk][experts]
+    size_t pf_moe_cap = 0;
+    float* pf_rlog = nullptr;
+    size_t pf_rlog_cap = 0;
     _Float16* pf_khl = nullptr;  // the prefill attention's K / V operands (f16 hi / lo keys, then f32 values)
     unsigned long long* pf_cells = nullptr;  // placement check of the XCD prefill attention
     int* pf_err = nullptr;
@@ -302,8 +333,8 @@ int moe_block_ffn(cmf_model_s* m, LayerDev& l, float* h, int nb, hipStream_t s) 
     const int H = c.hidden, ne = l.n_experts;
     if (l.router_f32) {
         hipLaunchKernelGGL(k_rms_rows, dim3(nb), dim3(256), 0, s, h, H, l.post_norm, H, c.eps, m->xrows);
-        hipLaunchKernelGGL(k_router_f32, dim3((ne + 3) / 4), dim3(256), 0, s, l.router_f32, m->xrows, ne, H, nb,
-                           m->rlog);
+        hipLaunchKernelGGL(k_router_f32, dim3((ne + 15) / 16, (nb + 15) / 16), dim3(1024), 0, s, l.router_f32, m->xrows,
+                           ne, H, nb, m->rlog);
         XSrc r{};
         r.mode = XS_ROWS;
         r.x = m->xrows;
@@ -563,6 +594,30 @@ int ensure_prefill_bufs(cmf_model_s* m) {
     return CMF_OK;
 }
 
+// The scratch of the routed-expert blocks' prefill: for the widest of them.
+int ensure_prefill_moe(cmf_model_s* m) {
+    const int R = std::min(prefill_chunk(), m->c.max_seq);
+    size_t need = 0, rl = 0;
+    for (auto& l : m->L)
+        if (l.moe) {
+            need = std::max(need, moe_prefill_scratch(l.moe, std::min(R, moe_prefill_tokens(l.moe))));
+            rl = std::max(rl, (size_t)R * l.n_experts);
+        }
+    auto grow = [&](void** p, size_t* cap, size_t bytes) -> int {
+        if (*cap >= bytes) return CMF_OK;
+        if (*p) {  // (a layer was replaced by a wider one)
+            m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), *p));
+            (void)hipFree(*p);
+            *p = nullptr;
+            *cap = 0;
+        }
+        if (dalloc(m, p, bytes)) return CMF_ERR;
+        *cap = bytes;
+        return CMF_OK;
+    };
+    return grow(&m->pf_moe, &m->pf_moe_cap, need) || grow((void**)&m->pf_rlog, &m->pf_rlog_cap, rl * sizeof(float)) ? CMF_ERR : CMF_OK;
+}
+
 // Causal attention of cnt chunk rows (positions *pb + i) in groups the
 // attention kernel serves (at most 32 queries per kv head); attend = 0 only
 // appends their K/V (the MTP warm).
@@ -590,6 +645,33 @@ void prefill_attention(cmf_model_s* m, LayerDev& l, const float* qkv, float* ao,
     }
 }
 
+// The routed-expert FFN over cnt > 16 prefill rows of h: the router on all
+// rows, then the experts' large-batch GEMMs (moe_prefill_launch), as many
+// tokens a call as it takes.  The 16-row batches of the verify kernels read
+// the experts' weights once per batch: 600 rows of the 128-expert 2048/768
+// layer took 9.6 ms.
+int prefill_moe(cmf_model_s* m, LayerDev& l, float* h, int cnt, hipStream_t s) {
+    const auto& c = m->c;
+    const int H = c.hidden, ne = l.n_experts, chunk = moe_prefill_tokens(l.moe);
+    XSrc x = src_norm(h, H, l.post_norm, c.eps);
+    if (l.router_f32) {
+        // (pf_hm: the MTP warm of the chunk comes after the layers)
+        hipLaunchKernelGGL(k_rms_rows, dim3(cnt), dim3(256), 0, s, h, H, l.post_norm, H, c.eps, m->pf_hm);
+        hipLaunchKernelGGL(k_router_f32, dim3((ne + 15) / 16, (cnt + 15) / 16), dim3(1024), 0, s, l.router_f32, m->pf_hm,
+                           ne, H, cnt, m->pf_rlog);
+    } else {
+        const int rc = gemm(l.router, x, cnt, m->pf_rlog, ne, false, s);
+        if (rc != CMF_OK) return rc;
+    }
+    for (int t0 = 0; t0 < cnt; t0 += chunk) {
+        x.x = h + (size_t)t0 * H;
+        const int rc = moe_prefill_launch(l.moe, x, m->pf_rlog + (size_t)t0 * ne, std::min(chunk, cnt - t0),
+                                          h + (size_t)t0 * H, H, true, m->pf_moe, s);
+        if (rc != CMF_OK) return rc;
+    }
+    return CMF_OK;
+}
+
 // One decoder block over a prefill chunk of cnt rows of h (forward_layers_span
 // over a batch, pipeline.rs:5100-5108 / 7981-8700) on the GEMMs: the
 // norm and SwiGLU producers prepare each GEMM's operand, the residual adds
@@ -605,7 +687,9 @@ int prefill_block(cmf_model_s* m, LayerDev& l, float* h, int cnt, const int* pb,
     ra.x = m->pf_ao;
     ra.ldx = nh * hd;
     if ((rc = gemm(l.wo, ra, cnt, h, H, true, s)) != CMF_OK) return rc;
-    if (l.moe) {  // the routed experts in batches of 16 rows (the verify-batch kernels)
+    if (l.moe) {
+        if (cnt > MAXB && moe_prefill_ok(l.moe, src_norm(h, H, l.post_norm, c.eps))) return prefill_moe(m, l, h, cnt, s);
+        // the routed experts in batches of 16 rows (the verify-batch kernels)
         for (int b0 = 0; b0 < cnt; b0 += MAXB)
             if ((rc = moe_block_ffn(m, l, h + (size_t)b0 * H, std::min(MAXB, cnt - b0), s))) return rc;
         return CMF_OK;
@@ -931,7 +1015,7 @@ static int ready(cmf_model m) {
 int cmf_prefill(cmf_model m, const int32_t* ids, int n) {
     if (ready(m)) return CMF_ERR;
     if (!ids || n < 1 || n + 1 > m->c.max_seq) return fail("prefill: 1 <= n < max_seq");
-    if (ensure_prefill_bufs(m)) return CMF_ERR;
+    if (ensure_prefill_bufs(m) || ensure_prefill_moe(m)) return CMF_ERR;
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= m->c.vocab) return fail("prefill: token id out of range");
     hipStream_t s = stream();

@@ -47,6 +47,11 @@ struct GemmArgs {
     // y written directly)
     int gsteps;
     float* part;
+    // grouped (MoE experts): batch tile y holds tiles[y].y <= 64 rows of
+    // expert tiles[y].x, whose weight is desc[tiles[y].x] (tiles == nullptr:
+    // one weight for all rows)
+    const int2* tiles;
+    const GemvDesc* desc;
 };
 
 constexpr int G4_NB = 3;           // k_gemm_q4: operand stages in LDS
@@ -96,6 +101,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_q4(GemmArgs a) {
     // load target the compiler waits for every load in flight before each
     // LDS read)
     extern __shared__ __align__(16) uint4 gemm_at[];
+    if (a.tiles) {  // (uniform)
+        const int2 t = a.tiles[blockIdx.y];
+        if (t.y == 0) return;
+        const GemvDesc d = a.desc[t.x];
+        a.w = d.w;
+        a.scale = d.scale;
+        a.rowp = d.rowp;
+        a.M = GB * (int)blockIdx.y + t.y;
+    }
     // q4tp: the 32 rungs of every row, rung c of row i in word c ^ (i % 32)
     // (rows' equal rungs in different banks)
     __shared__ float lad[TP ? 4 * RN * 32 * 32 : 1];
@@ -313,6 +327,15 @@ __global__ __launch_bounds__(256) void k_gemm_q8(GemmArgs a) {
     // double-buffered operand tile [2][Q8CH chunks][64 lanes] x 16 B, filled
     // by direct global -> LDS loads (as k_gemm_q4)
     extern __shared__ __align__(16) int4v gemm_at8[];
+    if (a.tiles) {  // (uniform)
+        const int2 t = a.tiles[blockIdx.y];
+        if (t.y == 0) return;
+        const GemvDesc d = a.desc[t.x];
+        a.w = d.w;
+        a.scale = d.scale;
+        a.rowp = d.rowp;
+        a.M = GB * (int)blockIdx.y + t.y;
+    }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, s = lane >> 4;
     const int by = blockIdx.y, rbw = (blockIdx.x * 4 + wave) * Q8RB;
@@ -461,6 +484,49 @@ static int gemm_kparts(long base, int nsteps) {
     return z;
 }
 
+// Allows kernel kf its dynamic LDS (once a kernel).
+static int gemm_lds(const void* kf, size_t bytes) {
+    static std::mutex mu;
+    static std::set<const void*> done;
+    std::lock_guard<std::mutex> g(mu);
+    if (!done.count(kf)) {
+        CMF_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+        done.insert(kf);
+    }
+    return CMF_OK;
+}
+
+// y[row][n] (ldy) of the rows of every tile, planes and xs prepared for
+// ntiles * 64 rows (proto: an expert's weight, for the shape and codec).
+// 64 weight rows a wave: the tiles alone fill the CUs.
+int gemm_grouped(const DevWeight& proto, const GemvDesc* desc, const int2* tiles, int ntiles, const uint8_t* planes,
+                 const float* xs, float* y, int ldy, hipStream_t st) {
+    if (ntiles < 1 || ntiles > 65535 || !desc || !tiles) return fail("gemm: bad tile list");
+    GemmArgs a{};
+    a.planes = planes;
+    a.xs = xs;
+    a.y = y;
+    a.ldy = ldy;
+    a.Mp = ntiles * GB;
+    a.N = proto.rows;
+    a.ntg = proto.kchunks;
+    a.nrb = proto.rows_pad / 16;
+    a.tiles = tiles;
+    a.desc = desc;
+    void* args[] = {&a};
+    if (proto.dtype == DT_Q8ROW) {
+        a.gsteps = (a.ntg + 1) / 2;
+        CMF_HIP(hipLaunchKernel((const void*)k_gemm_q8<2>, dim3((a.nrb + 7) / 8, ntiles), dim3(256), args,
+                                GEMM_Q8_AT_BYTES, st));
+        return CMF_OK;
+    }
+    a.gsteps = a.ntg;
+    const void* kf = proto.dtype == DT_Q4T ? (const void*)k_gemm_q4<DT_Q4T, 2> : (const void*)k_gemm_q4<DT_Q4TP, 2>;
+    if (gemm_lds(kf, GEMM_AT_BYTES) != CMF_OK) return CMF_ERR;
+    CMF_HIP(hipLaunchKernel(kf, dim3((a.nrb + 15) / 16, ntiles), dim3(256), args, GEMM_AT_BYTES, st));
+    return CMF_OK;
+}
+
 size_t gemm_planes_bytes(const DevWeight& w, int mp) {
     // q8: three planes of nk * 64 * Mp B; q4: hi + lo 2 * items * Mp * 16 B
     if (w.dtype == DT_Q8ROW) return (size_t)w.kchunks * 64 * mp * 3;
@@ -505,6 +571,8 @@ int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool res
     a.nrb = w.rows_pad / 16;
     a.resid = resid ? 1 : 0;
     a.part = nullptr;
+    a.tiles = nullptr;
+    a.desc = nullptr;
     // split K (nz parts into the partial buffer, then k_gemm_reduce)
     auto split = [&](long base, int nsteps) -> int {
         const int nz = gemm_kparts(base, nsteps);
@@ -552,14 +620,7 @@ int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool res
     const bool q4t = w.dtype == DT_Q4T;
     const void* kf = rn == 2 ? (q4t ? (const void*)k_gemm_q4<DT_Q4T, 2> : (const void*)k_gemm_q4<DT_Q4TP, 2>)
                              : (q4t ? (const void*)k_gemm_q4<DT_Q4T, 1> : (const void*)k_gemm_q4<DT_Q4TP, 1>);
-    {
-        // the operand tile's dynamic LDS is above the default 64 KiB limit
-        static std::mutex mu;
-        static std::set<const void*> done;
-        std::lock_guard<std::mutex> g(mu);
-        if (done.insert(kf).second)
-            CMF_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_AT_BYTES));
-    }
+    if (gemm_lds(kf, GEMM_AT_BYTES) != CMF_OK) return CMF_ERR;
     void* args[] = {&a};
     CMF_HIP(hipLaunchKernel(kf, grid, dim3(256), args, GEMM_AT_BYTES, st));
     return reduce(nz);

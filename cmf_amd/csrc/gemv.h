@@ -135,6 +135,17 @@ int launch_prep_rows_gemm(const DevWeight& w, const float* x, int ldx, int m, in
 // large-batch MFMA GEMM (gemm.hip) over the operand of the producer src
 // (XS_ROWS, XS_NORM, XS_SILU8, XS_CAT; resid: y += W x).
 int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st);
+// The same with a weight per batch tile of 64 rows (tiles: expert, rows in
+// use; unused tiles hold 0 rows) over prepared planes (launch_prep_gemm_map).
+int gemm_grouped(const DevWeight& proto, const GemvDesc* desc, const int2* tiles, int ntiles, const uint8_t* planes,
+                 const float* xs, float* y, int ldy, hipStream_t st);
+size_t gemm_planes_bytes(const DevWeight& w, int mp);
+// The GEMM operand of mp rows of which row b is wanted where map[b] >= 0,
+// made from row map[b] (gather) or b of src; prep_gemm_map_ok: whether the
+// producer has an instance for this source and weight.
+bool prep_gemm_map_ok(const DevWeight& w, const XSrc& src);
+int launch_prep_gemm_map(const DevWeight& w, const XSrc& src, const int* map, bool gather, int mp, uint8_t* planes,
+                         float* xs, hipStream_t st);
 // the same over plain device rows x [m][ldx]
 int gemm_q4(const DevWeight& w, const float* x, int ldx, int m, float* y, int ldy, hipStream_t st);
 // The same for up to max_jobs jobs of a device job list (GemvArgs::jobs):

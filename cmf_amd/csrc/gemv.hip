@@ -55,11 +55,18 @@ __global__ __launch_bounds__(512) void k_prep_src(XSrc s, int K, int fmt, int nk
 // ---------------------------------------------------------------------------
 template <bool Q8, int MODE, int NI>
 __global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, uint8_t* __restrict__ planes,
-                                                   float* __restrict__ xs, int Mp, int m) {
+                                                   float* __restrict__ xs, int Mp, int m,
+                                                   const int* __restrict__ map, int gather) {
     constexpr int C = Q8 ? 16 : 8;
-    const int lane = threadIdx.x & 63, b = blockIdx.x * 8 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, b = blockIdx.x * 8 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (b >= m) return;
-    const float* row = s.x + (size_t)b * s.ldx;
+    int sb = b;
+    if (map) {  // row b is made from row map[b] (gather) or b; none: map[b] < 0
+        const int t = map[b];
+        if (t < 0) return;
+        if (gather) sb = t;
+    }
+    const float* row = s.x + (size_t)sb * s.ldx;
     float v[NI][C];
     float4 wv[MODE == XS_NORM ? NI : 1][C / 4];
 #pragma unroll
@@ -154,7 +161,7 @@ __global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, ui
 
 // The instance that holds nitems per row (nullptr: none; the row's columns
 // per lane: up to 128)
-typedef void (*PrepGemm)(XSrc, int, int, uint8_t*, float*, int, int);
+typedef void (*PrepGemm)(XSrc, int, int, uint8_t*, float*, int, int, const int*, int);
 template <bool Q8, int MODE>
 static PrepGemm prep_gemm_pick(int nitems) {
     constexpr int D = Q8 ? 2 : 1;
@@ -345,7 +352,8 @@ int launch_prep_src_gemm(const DevWeight& w, const XSrc& src, int m, int mstride
     if (src.mode == XS_CAT && (src.H < 1 || src.H >= K)) return fail("prep: bad concat split");
     const int nk = w.dtype == DT_Q8ROW ? w.kchunks : w.kchunks * 4;
     if (PrepGemm pk = prep_gemm_kernel(w, src, K)) {
-        hipLaunchKernelGGL(pk, dim3((m + 7) / 8), dim3(512), 0, st, src, K, nk * 4, planes, xs, mstride, m);
+        hipLaunchKernelGGL(pk, dim3((m + 7) / 8), dim3(512), 0, st, src, K, nk * 4, planes, xs, mstride, m,
+                           (const int*)nullptr, 0);
         return CMF_OK;
     }
     // (256 threads a row: all of a 2048-row chunk's workgroups resident at
@@ -353,6 +361,21 @@ int launch_prep_src_gemm(const DevWeight& w, const XSrc& src, int m, int mstride
     // against 512, 12.5 ms at 128)
     hipLaunchKernelGGL(k_prep_src, dim3((m + 255) / 256 * 256), dim3(256), (size_t)K * sizeof(float), st, src, K,
                        w.dtype, nk, planes, xs, (const int*)nullptr, (size_t)0, (size_t)0, mstride, m);
+    return CMF_OK;
+}
+
+bool prep_gemm_map_ok(const DevWeight& w, const XSrc& src) {
+    const int K = src.K ? src.K : w.cols;
+    return K >= 1 && K <= w.cols && prep_gemm_kernel(w, src, K) != nullptr;
+}
+
+int launch_prep_gemm_map(const DevWeight& w, const XSrc& src, const int* map, bool gather, int mp, uint8_t* planes,
+                         float* xs, hipStream_t st) {
+    const int K = src.K ? src.K : w.cols;
+    PrepGemm pk = K >= 1 && K <= w.cols ? prep_gemm_kernel(w, src, K) : nullptr;
+    if (!pk || mp < 1 || mp % 64 || !map) return fail("prep: no mapped producer for this operand");
+    const int nk = w.dtype == DT_Q8ROW ? w.kchunks : w.kchunks * 4;
+    hipLaunchKernelGGL(pk, dim3(mp / 8), dim3(512), 0, st, src, K, nk * 4, planes, xs, mp, mp, map, gather ? 1 : 0);
     return CMF_OK;
 }
 

@@ -243,6 +243,100 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float* __restrict__ y
 }
 
 // ---------------------------------------------------------------------------
+// Prefill chunks (T > 16 tokens): the (token, rank) pairs sorted by expert
+// into rows of a large-batch GEMM whose 64-row batch tiles each belong to
+// one expert, so that an expert's weights are read once per tile instead of
+// once per 16-token batch.
+// ---------------------------------------------------------------------------
+// Routing of tokens 16 g .. of workgroup g, one wave each.
+__global__ __launch_bounds__(1024) void k_moe_route(const float* __restrict__ logits, int T, int ne, int k,
+                                                    int norm_topk, float scaling, int* __restrict__ idx,
+                                                    float* __restrict__ w) {
+    __shared__ int sidx[MAXB * MOE_MAX_TOPK];
+    __shared__ __align__(16) float pe[MAXB][MOE_MAX_EXPERTS];
+    const int t0 = blockIdx.x * MAXB, b = min(MAXB, T - t0);
+    logits += (size_t)t0 * ne;
+    idx += t0 * k;
+    w += t0 * k;
+    if (ne <= 64)
+        moe_route_tokens<1>(logits, b, ne, k, norm_topk, scaling, idx, w, sidx, pe);
+    else if (ne <= 128)
+        moe_route_tokens<2>(logits, b, ne, k, norm_topk, scaling, idx, w, sidx, pe);
+    else if (ne <= 256)
+        moe_route_tokens<4>(logits, b, ne, k, norm_topk, scaling, idx, w, sidx, pe);
+    else
+        moe_route_tokens<MOE_MAX_EXPERTS / 64>(logits, b, ne, k, norm_topk, scaling, idx, w, sidx, pe);
+}
+
+// The pairs' rows: expert e's pairs take the rows of ceil(count / 64) tiles
+// (their order within the expert is free: every row's result is its own).
+// slot[p] = row of pair p, rowmap[row] = its token or -1, tiles[i] =
+// (expert, rows in use), zero rows past the last.  One workgroup.
+__global__ __launch_bounds__(1024) void k_moe_group(const int* __restrict__ idx, int npairs, int ne, int k,
+                                                    int maxtiles, int* __restrict__ slot, int* __restrict__ rowmap,
+                                                    int2* __restrict__ tiles) {
+    __shared__ int cnt[MOE_MAX_EXPERTS], base[MOE_MAX_EXPERTS], wtot[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    cnt[tid] = 0;
+    for (int i = tid; i < maxtiles * 64; i += 1024) rowmap[i] = -1;
+    __syncthreads();
+    auto expert = [&](int p) { return min(max(idx[p], 0), ne - 1); };
+    for (int p = tid; p < npairs; p += 1024) atomicAdd(&cnt[expert(p)], 1);
+    __syncthreads();
+    const int c = tid < ne ? cnt[tid] : 0, nt = (c + 63) >> 6;
+    int inc = nt;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(inc, o);
+        if (lane >= o) inc += v;
+    }
+    if (lane == 63) wtot[wave] = inc;
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int i = 0; i < 16; i++) {
+        if (i < wave) before += wtot[i];
+        total += wtot[i];
+    }
+    const int b0 = before + inc - nt;
+    base[tid] = b0;
+    cnt[tid] = 0;
+    for (int j = 0; j < nt; j++) tiles[b0 + j] = make_int2(tid, min(64, c - 64 * j));
+    for (int i = total + tid; i < maxtiles; i += 1024) tiles[i] = make_int2(0, 0);
+    __syncthreads();
+    for (int p = tid; p < npairs; p += 1024) {
+        const int e = expert(p), row = (base[e] << 6) + atomicAdd(&cnt[e], 1);
+        slot[p] = row;
+        rowmap[row] = p / k;
+    }
+}
+
+// k_moe_combine over the pairs' rows: out[t] (+)= sum over ranks i in order
+// of w[t][i] * yd[slot[t k + i]].  grid (hidden / 1024, T), 256: four columns
+// a thread.
+__global__ __launch_bounds__(256) void k_moe_combine_rows(const float* __restrict__ yd, int ldy,
+                                                          const int* __restrict__ slot, const float* __restrict__ w,
+                                                          int k, int hidden, float* __restrict__ out, int ldo,
+                                                          int resid) {
+    const int t = blockIdx.y, h = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (h >= hidden) return;  // (hidden % 32 == 0)
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+    for (int i = 0; i < k; i++) {
+        const float4 v = *(const float4*)(yd + (size_t)slot[t * k + i] * ldy + h);
+        const float c = w[t * k + i];
+        acc.x += c * v.x;
+        acc.y += c * v.y;
+        acc.z += c * v.z;
+        acc.w += c * v.w;
+    }
+    float4* o = (float4*)(out + (size_t)t * ldo + h);
+    if (resid) {
+        const float4 r = *o;
+        acc = make_float4(r.x + acc.x, r.y + acc.y, r.z + acc.z, r.w + acc.w);
+    }
+    *o = acc;
+}
+
+// ---------------------------------------------------------------------------
 // q4t expert GEMVs over the job's own tokens.  Job j (grid.y) multiplies
 // expert desc[jobs[1 + j]] with the n <= 8 token rows of its list jt[j]
 // only: the other tokens of the batch cost no operand traffic and no LDS.
@@ -861,6 +955,74 @@ int cmf::moe_ffn_launch(cmf_moe m, const XSrc& x, const float* d_logits, int b, 
                        m->ne, m->top_k, m->norm_topk, m->scaling, m->idx, m->w, m->jobs, m->slot, m->jt, x, K,
                        g.dtype, nk, m->px, m->xsx);
     return moe_experts(m, x, b, m->top_k, d_out, ldo, resid, s, true, true);
+}
+
+// Prefill rows: at most 16384 pairs a call (config-5 experts: 24576 rows with
+// the tiles' padding, 200 MB of operand planes and 350 of outputs; more
+// rows a call would no longer save weight reads).
+int cmf::moe_prefill_tokens(cmf_moe m) { return std::max(MAXB, 16384 / m->top_k); }
+static int moe_prefill_maxtiles(cmf_moe m, int T) {
+    const int pairs = T * m->top_k;
+    return pairs / 64 + std::min(m->ne, pairs);
+}
+namespace {
+struct MoeRows {  // the scratch of one call
+    int *idx, *slot, *rowmap;
+    float *w, *xs, *y;
+    int2* tiles;
+    uint8_t* planes;
+    size_t bytes;
+    MoeRows(cmf_moe m, int T, void* p) {
+        const int mt = moe_prefill_maxtiles(m, T), pairs = T * m->top_k;
+        const size_t rows = (size_t)mt * 64;
+        size_t at = 0;
+        auto take = [&](size_t n) {
+            void* q = (char*)p + at;
+            at += (n + 255) & ~(size_t)255;
+            return q;
+        };
+        idx = (int*)take(sizeof(int) * pairs);
+        slot = (int*)take(sizeof(int) * pairs);
+        w = (float*)take(sizeof(float) * pairs);
+        rowmap = (int*)take(sizeof(int) * rows);
+        tiles = (int2*)take(sizeof(int2) * mt);
+        xs = (float*)take(sizeof(float) * rows);
+        planes = (uint8_t*)take(std::max(gemm_planes_bytes(m->gu[0], (int)rows), gemm_planes_bytes(m->down[0], (int)rows)));
+        // gate|up outputs, then (once the down operand is made) the down outputs
+        y = (float*)take(sizeof(float) * rows * std::max(2 * m->inter, m->hidden));
+        bytes = at;
+    }
+};
+XSrc moe_h_src(cmf_moe m, const float* gu) {
+    XSrc s{};
+    s.mode = XS_SILU8;  // (gate|up rows interleaved 8 / 8)
+    s.x = gu;
+    s.ldx = 2 * m->inter;
+    s.K = m->inter;
+    return s;
+}
+}  // namespace
+size_t cmf::moe_prefill_scratch(cmf_moe m, int T) { return MoeRows(m, T, nullptr).bytes; }
+bool cmf::moe_prefill_ok(cmf_moe m, const XSrc& x) {
+    return m->hidden % 4 == 0 && prep_gemm_map_ok(m->gu[0], x) && prep_gemm_map_ok(m->down[0], moe_h_src(m, nullptr));
+}
+int cmf::moe_prefill_launch(cmf_moe m, const XSrc& x, const float* d_logits, int T, float* d_out, int ldo, bool resid,
+                            void* scratch, hipStream_t s) {
+    if (T < 1 || T > moe_prefill_tokens(m)) return fail("moe: too many prefill rows");
+    if (ldo % 4 || (uintptr_t)d_out % 16) return fail("moe: prefill output rows must be 16-byte aligned");
+    const int H = m->hidden, I = m->inter, k = m->top_k, mt = moe_prefill_maxtiles(m, T);
+    const MoeRows r(m, T, scratch);
+    hipLaunchKernelGGL(k_moe_route, dim3((T + MAXB - 1) / MAXB), dim3(64 * MAXB), 0, s, d_logits, T, m->ne, k,
+                       m->norm_topk, m->scaling, r.idx, r.w);
+    hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(1024), 0, s, r.idx, T * k, m->ne, k, mt, r.slot, r.rowmap, r.tiles);
+    int rc = launch_prep_gemm_map(m->gu[0], x, r.rowmap, true, mt * 64, r.planes, r.xs, s);
+    if (rc == CMF_OK) rc = gemm_grouped(m->gu[0], m->d_gu, r.tiles, mt, r.planes, r.xs, r.y, 2 * I, s);
+    if (rc == CMF_OK) rc = launch_prep_gemm_map(m->down[0], moe_h_src(m, r.y), r.rowmap, false, mt * 64, r.planes, r.xs, s);
+    if (rc == CMF_OK) rc = gemm_grouped(m->down[0], m->d_down, r.tiles, mt, r.planes, r.xs, r.y, H, s);
+    if (rc != CMF_OK) return rc;
+    hipLaunchKernelGGL(k_moe_combine_rows, dim3((H + 1023) / 1024, T), dim3(256), 0, s, r.y, H, r.slot, r.w, k, H,
+                       d_out, ldo, resid ? 1 : 0);
+    return CMF_OK;
 }
 
 extern "C" {

@@ -44,5 +44,14 @@ int moe_hidden(cmf_moe_s* m);
 int moe_experts_count(cmf_moe_s* m);
 int moe_ffn_launch(cmf_moe_s* m, const XSrc& x, const float* d_logits, int b, float* d_out, int ldo, bool resid,
                    hipStream_t s);
+// The same for T > 16 rows (a prefill chunk): every (token, expert) pair in
+// expert order through the large-batch GEMMs.  scratch:
+// moe_prefill_scratch(m, T) bytes; moe_prefill_ok: whether the layer's
+// operands have a producer (else the rows go 16 at a time).
+int moe_prefill_tokens(cmf_moe_s* m);  // the most rows of one call
+size_t moe_prefill_scratch(cmf_moe_s* m, int T);
+bool moe_prefill_ok(cmf_moe_s* m, const XSrc& x);
+int moe_prefill_launch(cmf_moe_s* m, const XSrc& x, const float* d_logits, int T, float* d_out, int ldo, bool resid,
+                       void* scratch, hipStream_t s);
 
 }  // namespace cmf
