@@ -533,7 +533,7 @@ size_t gemm_planes_bytes(const DevWeight& w, int mp) {
     return (size_t)w.kchunks * 16 * mp * 32;
 }
 
-int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st) {
+int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st, bool prepared) {
     if (w.dtype != DT_Q4T && w.dtype != DT_Q4TP && w.dtype != DT_Q8ROW) return fail("gemm: q8 / q4t / q4tp weights");
     if (m < 1 || m > 65535) return fail("gemm: batch must be 1..65535");
     const int mp = (m + GB - 1) / GB * GB;
@@ -554,8 +554,10 @@ int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool res
         CMF_HIP(hipMalloc(&g_gemm_xs, (size_t)mp * sizeof(float)));
         g_gemm_xs_cap = mp;
     }
-    int rc = launch_prep_src_gemm(w, src, m, mp, g_gemm_planes, g_gemm_xs, st);
-    if (rc != CMF_OK) return rc;
+    if (!prepared) {
+        const int rc = launch_prep_src_gemm(w, src, m, mp, g_gemm_planes, g_gemm_xs, st);
+        if (rc != CMF_OK) return rc;
+    }
     GemmArgs a;
     a.w = w.w;
     a.scale = w.scale;

@@ -97,6 +97,7 @@ GemvKernel q8_kernel(int m, int xm, int ks);
 // k_gemv_q4t_m1): the instance, its waves per workgroup (*ks) and dynamic
 // LDS bytes (*lds), or nullptr
 GemvKernel q8_kernel_m1(int nk, bool resid, int* ks, size_t* lds);
+GemvKernel q8_kernel_m1x(int nk, bool resid, int* ks);
 GemvKernel q4t_kernel_m1(int nk, bool resid, int* ks, size_t* lds);
 // q4t, M = 1, the operand staged from its f32 row inside the kernel (XS_ROWS)
 GemvKernel q4t_kernel_m1x(int nk, bool resid, int* ks);
@@ -133,8 +134,10 @@ int launch_prep_rows_gemm(const DevWeight& w, const float* x, int ldx, int m, in
                           float* xs, hipStream_t st);
 // y[b][n] (ldy) (+)= W x[b] for b < m, any m, q8 / q4t / q4tp weights: the
 // large-batch MFMA GEMM (gemm.hip) over the operand of the producer src
-// (XS_ROWS, XS_NORM, XS_SILU8, XS_CAT; resid: y += W x).
-int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st);
+// (XS_ROWS, XS_NORM, XS_SILU, XS_SILU8, XS_CAT; resid: y += W x).  prepared:
+// the operand is the one of the thread's last gemm() (same codec and columns).
+int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool resid, hipStream_t st,
+         bool prepared = false);
 // The same with a weight per batch tile of 64 rows (tiles: expert, rows in
 // use; unused tiles hold 0 rows) over prepared planes (launch_prep_gemm_map).
 int gemm_grouped(const DevWeight& proto, const GemvDesc* desc, const int2* tiles, int ntiles, const uint8_t* planes,
@@ -155,6 +158,9 @@ int launch_prep_src_grouped(const DevWeight& w, const XSrc& src, int m, const in
                             size_t x_stride, uint8_t* planes, size_t planes_stride, float* xs, hipStream_t st);
 int launch_prep(const DevWeight& w, const float* x, int ldx, int m, uint8_t* planes, float* xs,
                 hipStream_t st);
+// Whether gemv() of one plain f32 row x runs as one launch that stages its
+// own operand slices (k_gemv_q4t_m1x, k_gemv_q8_m1x).
+bool gemv_m1x_ok(const DevWeight& w, const float* x);
 // The a8w8 operand (split_act) of m rows of x: planes / xs as launch_prep,
 // plus the outlier lists in o (cap >= w.cols).
 int launch_prep_a8(const DevWeight& w, const float* x, int ldx, int m, uint8_t* planes, float* xs, const A8Out& o,
@@ -167,13 +173,16 @@ int gemv_a8(const DevWeight& w, const uint8_t* planes, const float* xs, const A8
 int launch_gemv(const DevWeight& w, const uint8_t* planes, const float* xs, float* y, int ldy,
                 int m, int row_lo, int row_hi, hipStream_t st, int ks_override = 0);
 
-// x ~= q0 + q1/128 + q2/16384 (each int8, |error| <= 2^-22 * 127), the
-// three bytes or-ed into byte j of a, b, c.  v = x / (amax / 127) lies
+// x / sx ~= q0 + q1/128 + q2/16384 (each int8, |error| <= 2^-22 * 127; inv =
+// 1 / sx), the three bytes or-ed into byte j of a, b, c.  v = x * inv lies
 // within 127 * (1 + 2^-22) of zero, so rint(v) is in [-127, 127] and the
-// remainders (v - q0) * 128 and (r1 - q1) * 128 in [-64, 64]: no clamps.
-__device__ __forceinline__ void q8_split(float v, int j, uint32_t& a, uint32_t& b, uint32_t& c) {
-    const float q0 = rintf(v);
-    const float r1 = (v - q0) * 128.0f;
+// remainders (v - q0) * 128 and (r1 - q1) * 128 round to [-64, 64]: no
+// clamps.  The first remainder is one FMA by name, so that every kernel that
+// makes these planes makes the same ones (left to the compiler, some fused
+// it and some did not).
+__device__ __forceinline__ void q8_split(float x, float inv, int j, uint32_t& a, uint32_t& b, uint32_t& c) {
+    const float q0 = rintf(x * inv);
+    const float r1 = __builtin_fmaf(x, inv, -q0) * 128.0f;
     const float q1 = rintf(r1);
     const float r2 = (r1 - q1) * 128.0f;
     const float q2 = rintf(r2);
@@ -202,7 +211,7 @@ __device__ inline void prep8_row(const float* x, int K, float amax, int nk, int 
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int col = c0 + 4 * q + j;
-                q8_split(col < K ? x[col] * inv : 0.f, j, a, bb, c);
+                q8_split(col < K ? x[col] : 0.f, inv, j, a, bb, c);
             }
             w0[q] = a;
             w1[q] = bb;
@@ -350,10 +359,10 @@ __device__ inline void prep8_rows(const float* raw, int K, const float* amv, int
             // K % 4 == 0: a unit is all inside or all past the row
             const float4 xv = c0 < K ? *(const float4*)(raw + (size_t)b * K + c0) : make_float4(0.f, 0.f, 0.f, 0.f);
             uint32_t a = 0, bb = 0, c = 0;
-            q8_split(xv.x * inv, 0, a, bb, c);
-            q8_split(xv.y * inv, 1, a, bb, c);
-            q8_split(xv.z * inv, 2, a, bb, c);
-            q8_split(xv.w * inv, 3, a, bb, c);
+            q8_split(xv.x, inv, 0, a, bb, c);
+            q8_split(xv.y, inv, 1, a, bb, c);
+            q8_split(xv.z, inv, 2, a, bb, c);
+            q8_split(xv.w, inv, 3, a, bb, c);
             const size_t off = ((size_t)idx * m + b) * 16 + 4 * q4;
             *(uint32_t*)(p0 + off) = a;
             *(uint32_t*)(p1 + off) = bb;
@@ -376,10 +385,10 @@ __device__ inline void prep8_rows(const float* raw, int K, const float* amv, int
             const int c = c0 + 4 * q4;
             const float4 xv = c < K ? *(const float4*)(raw + (size_t)b * K + c) : make_float4(0.f, 0.f, 0.f, 0.f);
             uint32_t a = 0, bb = 0, cc = 0;
-            q8_split(xv.x * inv, 0, a, bb, cc);
-            q8_split(xv.y * inv, 1, a, bb, cc);
-            q8_split(xv.z * inv, 2, a, bb, cc);
-            q8_split(xv.w * inv, 3, a, bb, cc);
+            q8_split(xv.x, inv, 0, a, bb, cc);
+            q8_split(xv.y, inv, 1, a, bb, cc);
+            q8_split(xv.z, inv, 2, a, bb, cc);
+            q8_split(xv.w, inv, 3, a, bb, cc);
             *(uint32_t*)(p0 + off + 4 * q4) = a;
             *(uint32_t*)(p1 + off + 4 * q4) = bb;
             *(uint32_t*)(p2 + off + 4 * q4) = cc;

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, ui
             if (idx >= nitems) continue;
             uint32_t w0[4] = {}, w1[4] = {}, w2[4] = {};
 #pragma unroll
-            for (int j = 0; j < 16; j++) q8_split(v[i][j] * inv, j & 3, w0[j >> 2], w1[j >> 2], w2[j >> 2]);
+            for (int j = 0; j < 16; j++) q8_split(v[i][j], inv, j & 3, w0[j >> 2], w1[j >> 2], w2[j >> 2]);
             uint8_t* p = planes + ((size_t)idx * Mp + b) * 16;
             *(uint4*)p = make_uint4(w0[0], w0[1], w0[2], w0[3]);
             *(uint4*)(p + plane) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, ui
 }
 
 // The instance that holds nitems per row (nullptr: none; the row's columns
-// per lane: up to 128)
+// per lane: up to 192)
 typedef void (*PrepGemm)(XSrc, int, int, uint8_t*, float*, int, int, const int*, int);
 template <bool Q8, int MODE>
 static PrepGemm prep_gemm_pick(int nitems) {
@@ -173,6 +173,8 @@ static PrepGemm prep_gemm_pick(int nitems) {
     if constexpr (MODE != XS_NORM) {  // (a norm's weights would spill past 64 columns per lane)
         if (ni <= 12) return k_prep_gemm<Q8, MODE, 12 / D>;
         if (ni <= 16) return k_prep_gemm<Q8, MODE, 16 / D>;
+        if constexpr (MODE != XS_SILU8)
+            if (ni <= 24) return k_prep_gemm<Q8, MODE, 24 / D>;
     }
     return nullptr;
 }
@@ -191,6 +193,133 @@ static PrepGemm prep_gemm_kernel(const DevWeight& w, const XSrc& s, int K) {
             return q8 ? prep_gemm_pick<true, XS_SILU>(nitems) : prep_gemm_pick<false, XS_SILU>(nitems);
         case XS_SILU8:
             return q8 ? prep_gemm_pick<true, XS_SILU8>(nitems) : prep_gemm_pick<false, XS_SILU8>(nitems);
+        default: return nullptr;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// GEMV operand of m <= 16 rows, split over workgroups: workgroup (b, y)
+// reduces the whole of row b (sum of squares, max|x|; the row comes from L2
+// after the first) and writes items [256 y, 256 (y + 1)) of its planes, one
+// per thread, so that a long row's quantisation is spread over the chip
+// instead of one workgroup.  Latency-bound: two memory round trips and one
+// or two barriers.  Values as prep_src_row's (f64 sums in another order).
+// Measured on MI355X (traced): 5 rows of 4096 10 -> 4.6 us, SwiGLU rows of
+// 12288 18 -> 7.4, 13 rows of 12288 13.6 -> 5.5.  grid (m, items / 256), 256.
+// ---------------------------------------------------------------------------
+template <bool Q8, int MODE>
+__global__ __launch_bounds__(256) void k_prep_split(XSrc s, int K, int nitems, uint8_t* __restrict__ planes,
+                                                    float* __restrict__ xs) {
+    constexpr int C = Q8 ? 16 : 8;
+    __shared__ double red[4];
+    __shared__ float redm[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x, M = gridDim.x;
+    const float* row = s.x + (size_t)b * s.ldx;
+    // four columns from c (K % 4 == 0: all inside the row or none)
+    auto val = [&](int c) __attribute__((always_inline)) -> float4 {
+        if constexpr (MODE == XS_SILU || MODE == XS_SILU8) {
+            const float* gp = MODE == XS_SILU ? row + c : row + 16 * (c >> 3) + (c & 7);
+            const float4 g = *(const float4*)gp, u = *(const float4*)(gp + (MODE == XS_SILU ? s.K : 8));
+            return make_float4((g.x / (1.0f + expf(-g.x))) * u.x, (g.y / (1.0f + expf(-g.y))) * u.y,
+                               (g.z / (1.0f + expf(-g.z))) * u.z, (g.w / (1.0f + expf(-g.w))) * u.w);
+        } else {
+            return *(const float4*)(row + c);
+        }
+    };
+    auto amax4 = [](float a, float4 v) { return fmaxf(fmaxf(a, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w))); };
+    float am = 0.f, inv = 1.f;
+    auto normed = [&](float4 v, int c) __attribute__((always_inline)) -> float4 {
+        if constexpr (MODE == XS_NORM) {
+            const float4 w = *(const float4*)(s.w + c);
+            return make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+        }
+        return v;
+    };
+    if constexpr (MODE == XS_NORM) {
+        double ss = 0.0;
+#pragma unroll 4
+        for (int c = 4 * tid; c < K; c += 1024) {
+            const float4 v = val(c);
+            ss += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+        __syncthreads();
+        inv = 1.0f / (float)sqrt((red[0] + red[1] + red[2] + red[3]) / (double)K + s.eps);
+    }
+#pragma unroll 4
+    for (int c = 4 * tid; c < K; c += 1024) am = amax4(am, normed(val(c), c));
+    am = wave_max(am);
+    if (lane == 0) redm[wave] = am;
+    // this thread's item (requested before the barrier)
+    const int idx = blockIdx.y * 256 + tid, c0 = idx * C;
+    float v[C];
+#pragma unroll
+    for (int q = 0; q < C / 4; q++) {
+        const bool in = idx < nitems && c0 + 4 * q < K;
+        const int c = in ? c0 + 4 * q : 0;
+        const float4 y = normed(val(c), c);
+        v[4 * q] = in ? y.x : 0.f;
+        v[4 * q + 1] = in ? y.y : 0.f;
+        v[4 * q + 2] = in ? y.z : 0.f;
+        v[4 * q + 3] = in ? y.w : 0.f;
+    }
+    __syncthreads();
+    am = fmaxf(fmaxf(redm[0], redm[1]), fmaxf(redm[2], redm[3]));
+    const bool on = idx < nitems;
+    uint8_t* p = planes + ((size_t)(on ? idx : 0) * M + b) * 16;
+    const size_t plane = (size_t)nitems * M * 16;
+    if constexpr (Q8) {
+        const float sx = am > 0.f ? am / 127.0f : 1.0f, is = 1.0f / sx;
+        if (idx == 0) xs[b] = sx;
+        uint32_t w0[4] = {}, w1[4] = {}, w2[4] = {};
+#pragma unroll
+        for (int j = 0; j < 16; j++) q8_split(v[j], is, j & 3, w0[j >> 2], w1[j >> 2], w2[j >> 2]);
+        if (!on) return;
+        *(uint4*)p = make_uint4(w0[0], w0[1], w0[2], w0[3]);
+        *(uint4*)(p + plane) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
+        *(uint4*)(p + 2 * plane) = make_uint4(w2[0], w2[1], w2[2], w2[3]);
+    } else {
+        float scale, xsv;
+        q4_fix_scale(am, scale, xsv);
+        if (idx == 0) xs[b] = xsv;
+        constexpr int ord[8] = {0, 4, 2, 6, 1, 5, 3, 7};
+        uint32_t hv[4] = {}, lv[4] = {};
+        float sh = 0.f, sl = 0.f;  // (exact: integers and multiples of 2^-11)
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            _Float16 h, l;
+            q4_fix_split(v[ord[j]] * scale, h, l);
+            hv[j >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, h) << (16 * (j & 1));
+            lv[j >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, l) << (16 * (j & 1));
+            sh += (float)h;
+            sl += (float)l;
+        }
+        sh += __shfl_xor(sh, 1);
+        sh += __shfl_xor(sh, 2);
+        sl += __shfl_xor(sl, 1);
+        sl += __shfl_xor(sl, 2);
+        if (!on) return;
+        *(uint4*)p = make_uint4(hv[0], hv[1], hv[2], hv[3]);
+        *(uint4*)(p + plane) = make_uint4(lv[0], lv[1], lv[2], lv[3]);
+        if ((idx & 3) == 0) q4_put_bias((float*)(planes + 2 * plane), nitems / 4, 16, M, idx >> 2, b, sh, sl);
+    }
+}
+
+// The split producer of src (nullptr: none for this mode or alignment)
+typedef void (*PrepSplit)(XSrc, int, int, uint8_t*, float*);
+static PrepSplit prep_split_kernel(const DevWeight& w, const XSrc& s, int K) {
+    const bool q8 = w.dtype == DT_Q8ROW;
+    if (K % 4 || s.ldx % 4 || (uintptr_t)s.x % 16) return nullptr;
+    switch (s.mode) {
+        case XS_ROWS: return q8 ? k_prep_split<true, XS_ROWS> : k_prep_split<false, XS_ROWS>;
+        case XS_NORM:
+            if ((uintptr_t)s.w % 16) return nullptr;
+            return q8 ? k_prep_split<true, XS_NORM> : k_prep_split<false, XS_NORM>;
+        case XS_SILU:
+            if (s.K % 4) return nullptr;
+            return q8 ? k_prep_split<true, XS_SILU> : k_prep_split<false, XS_SILU>;
+        case XS_SILU8: return q8 ? k_prep_split<true, XS_SILU8> : k_prep_split<false, XS_SILU8>;
         default: return nullptr;
     }
 }
@@ -338,6 +467,10 @@ int launch_prep_src(const DevWeight& w, const XSrc& src, int m, uint8_t* planes,
     if (K < 1 || K > w.cols || K > 16384) return fail("prep: operand length must be 1..min(cols, 16384)");
     if (src.mode == XS_CAT && (src.H < 1 || src.H >= K)) return fail("prep: bad concat split");
     const int nk = w.dtype == DT_Q8ROW ? w.kchunks : w.kchunks * 4;
+    if (PrepSplit ps = prep_split_kernel(w, src, K)) {
+        hipLaunchKernelGGL(ps, dim3(m, (nk * 4 + 255) / 256), dim3(256), 0, st, src, K, nk * 4, planes, xs);
+        return CMF_OK;
+    }
     hipLaunchKernelGGL(k_prep_src, dim3(m), dim3(512), (size_t)K * sizeof(float), st, src, K, w.dtype, nk, planes,
                        xs, (const int*)nullptr, (size_t)0, (size_t)0, 0, m);
     return CMF_OK;
@@ -502,6 +635,17 @@ static int pick_ks(int nk) {
     return k;
 }
 
+bool gemv_m1x_ok(const DevWeight& w, const float* x) {
+    static const int env = env_int("CMF_GEMV_M1X", 1);
+    XSrc s{};
+    s.mode = XS_ROWS;
+    s.x = x;
+    s.ldx = w.cols;
+    int ks = 0;
+    if (!env || fused_lds_bytes(w, s, 1) == 0) return false;
+    return w.dtype == DT_Q4T ? w.cols % 8 == 0 && q4t_kernel_m1x(w.kchunks, false, &ks) : w.dtype == DT_Q8ROW && q8_kernel_m1x(w.kchunks, false, &ks);
+}
+
 constexpr int FUSED_MIN_KS = 8;  // waves of a workgroup that stages m > 2 rows
 
 // Whether evaluating the producer inside the GEMV workgroups beats a
@@ -571,13 +715,14 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
             return CMF_OK;
         }
     }
-    // q4t M = 1 from the f32 row (XS_ROWS): the kernel that stages its own
-    // operand slices (CMF_GEMV_M1X=0 keeps the general fused kernel)
+    // M = 1 from the f32 row (XS_ROWS; q4t, q8): the kernels that stage
+    // their own operand slices (CMF_GEMV_M1X=0 keeps the general fused kernel)
     static const int m1x_env = env_int("CMF_GEMV_M1X", 1);
-    if (m1x_env && m == 1 && xm == XM_FUSED && a.src.mode == XS_ROWS && w.dtype == DT_Q4T && !grouped &&
-        grid_override <= 0 && ks_override <= 0 && a.epi == EPI_NONE && a.src.K % 8 == 0) {
+    if (m1x_env && m == 1 && xm == XM_FUSED && a.src.mode == XS_ROWS && (w.dtype == DT_Q4T || w.dtype == DT_Q8ROW) &&
+        !grouped && grid_override <= 0 && ks_override <= 0 && a.epi == EPI_NONE &&
+        (w.dtype == DT_Q8ROW || a.src.K % 8 == 0)) {
         int ks1 = 0;
-        GemvKernel k1 = q4t_kernel_m1x(w.kchunks, a.resid, &ks1);
+        GemvKernel k1 = w.dtype == DT_Q4T ? q4t_kernel_m1x(w.kchunks, a.resid, &ks1) : q8_kernel_m1x(w.kchunks, a.resid, &ks1);
         if (k1 && resident_per_cu(k1, 64 * ks1, 0) >= 1) {
             void* args[] = {&a};
             CMF_HIP(hipLaunchKernel((const void*)k1, dim3(a.nrb), dim3(64 * ks1), args, 0, st));

@@ -1176,6 +1176,90 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
     }
 }
 
+// q8, M = 1, from the f32 operand row itself (XS_ROWS), as k_gemv_q4t_m1x:
+// wave w reads the SPW * 64 columns of its own steps (four columns per lane
+// and pass), the workgroup agrees on the row's max |x| (one LDS exchange, the
+// weights in flight), each wave writes its slice's three int8 planes (the
+// producer's values) into its own LDS region and runs the MFMA loop of
+// k_gemv_q8_m1, whose per-wave sums are exact: equal to producer +
+// k_gemv_q8_m1 bit for bit.  Latency-bound: 1024x1024 producer launch + GEMV
+// 6.4 us a call, this 3.7.  K % 4 == 0; columns past K are zero.
+template <int KS, int SPW, bool RESID>
+__global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
+    constexpr int NIT = (SPW * 16 + 63) / 64;  // 4-column pieces per lane
+    __shared__ float part[KS][64];
+    __shared__ float wmax[KS];
+    // item i = (u * 4 + s') * 3 + p: plane p of step u, k-slot s'
+    __shared__ __align__(16) uint32_t slice[KS][SPW * 4 * 3 * 4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, s = lane >> 4;
+    const int nkc = a.nk, rb = blockIdx.x, K = a.src.K, c0 = wave * SPW;
+    const int row = (a.rb0 + rb) * 16 + r;
+    const int rowc = max(a.row_lo, min(row, a.row_hi - 1));
+    const float rs = ldg((const float*)a.scale + row);
+    const float yold = RESID ? ldg(a.y + (rowc - a.row_lo)) : 0.f;
+    float4v xv[NIT];
+    bool on[NIT];
+#pragma unroll
+    for (int i = 0; i < NIT; i++) {
+        const int q = lane + 64 * i, c = c0 * 64 + 4 * q;
+        on[i] = q < SPW * 16 && c < K;
+        xv[i] = ldg((const float4v*)(a.src.x + (on[i] ? c : 0)));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int4v wv[SPW];
+    const size_t wbase = (size_t)(a.rb0 + rb) * nkc;
+#pragma unroll
+    for (int u = 0; u < SPW; u++) wv[u] = ldg((const int4v*)a.w + (wbase + min(c0 + u, nkc - 1)) * 64 + lane);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<SPW>();  // this wave's operand columns are in
+    float am = 0.f;
+#pragma unroll
+    for (int i = 0; i < NIT; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) am = fmaxf(am, on[i] ? fabsf(xv[i][k]) : 0.f);
+    am = wave_max(am);
+    if (lane == 0) wmax[wave] = am;
+    // LDS-only barrier: the weights stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    am = wmax[0];
+#pragma unroll
+    for (int w = 1; w < KS; w++) am = fmaxf(am, wmax[w]);
+    const float xs = am > 0.f ? am / 127.0f : 1.0f;
+    const float inv = 1.0f / xs;
+#pragma unroll
+    for (int i = 0; i < NIT; i++) {
+        const int q = lane + 64 * i;
+        uint32_t b0 = 0, b1 = 0, b2 = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) q8_split(on[i] ? xv[i][k] : 0.f, inv, k, b0, b1, b2);
+        if (q < SPW * 16) {
+            uint32_t* d = slice[wave] + (q >> 2) * 12 + (q & 3);
+            d[0] = b0;
+            d[4] = b1;
+            d[8] = b2;
+        }
+    }
+    // (the wave reads back what its own lanes wrote, as k_gemv_q4t_m1x)
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int4v* X = (const int4v*)slice[wave];
+    int4v acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < SPW; u++) {
+        const int4v z = {0, 0, 0, 0};
+        const int4v xq = X[(u * 4 + s) * 3 + min(r, 2)];
+        const int4v xa = (r < 3 && c0 + u < nkc) ? xq : z;
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa, wv[u], acc, 0, 0, 0);
+    }
+    const float v = (float)acc[0] + (float)acc[1] * 0.0078125f + (float)acc[2] * 6.103515625e-05f;
+    const float o = m1_reduce<KS>(part, v, wave, lane);
+    if (wave == 0 && s == 0 && row >= a.row_lo && row < a.row_hi && rb < a.nrb) {
+        const float val = (o * xs) * rs;
+        a.y[row - a.row_lo] = RESID ? yold + val : val;
+    }
+}
+
 // Instance of the M = 1 kernels for rows of nk 1 KiB steps (nullptr: none);
 // *ks = its waves per workgroup, *lds = its dynamic LDS bytes.
 template <int KS, int SPW>
@@ -1202,6 +1286,21 @@ inline GemvKernel q8_m1_pick(int nk, bool resid, int* ks, size_t* lds) {
     if (nk <= 64) return q8_m1_inst<16, 4>(resid, ks, lds);
     if (nk <= 128) return q8_m1_inst<16, 8>(resid, ks, lds);
     if (nk <= 192) return q8_m1_inst<16, 12>(resid, ks, lds);
+    return nullptr;
+}
+template <int KS, int SPW>
+inline GemvKernel q8_m1x_inst(bool resid, int* ks) {
+    *ks = KS;
+    return resid ? k_gemv_q8_m1x<KS, SPW, true> : k_gemv_q8_m1x<KS, SPW, false>;
+}
+// (the waves and steps of q8_m1_pick, so that the sums are the same)
+inline GemvKernel q8_m1x_pick(int nk, bool resid, int* ks) {
+    if (nk <= 8) return q8_m1x_inst<1, 8>(resid, ks);
+    if (nk <= 16) return q8_m1x_inst<8, 2>(resid, ks);
+    if (nk <= 32) return q8_m1x_inst<8, 4>(resid, ks);
+    if (nk <= 64) return q8_m1x_inst<16, 4>(resid, ks);
+    if (nk <= 128) return q8_m1x_inst<16, 8>(resid, ks);
+    if (nk <= 192) return q8_m1x_inst<16, 12>(resid, ks);
     return nullptr;
 }
 template <int KS, int SPW>

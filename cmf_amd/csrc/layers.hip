@@ -260,8 +260,8 @@ __global__ __launch_bounds__(64) void k_attn_merge(AttnArgs a) {
     const float sx = am > 0.f ? am / 127.0f : 1.0f;
     const float inv = 1.0f / sx;
     uint32_t p0 = 0, p1 = 0, p2 = 0;
-    q8_split(o.x * inv, 0, p0, p1, p2);
-    q8_split(o.y * inv, 1, p0, p1, p2);
+    q8_split(o.x, inv, 0, p0, p1, p2);
+    q8_split(o.y, inv, 1, p0, p1, p2);
     const int cc = 2 * h + (lane >> 5), j = (2 * lane) & 63;
     const size_t off = ((size_t)(4 * cc + (j >> 4)) * M + br) * 16 + (j & 15);
     *(uint16_t*)(a.wop + off) = (uint16_t)p0;

@@ -327,8 +327,7 @@ int seam_matmat(const DevWeight& w_in, int row0, const float* xs, int b, int row
         const int m = std::min(MAXB, b - b0);
         CMF_HIP(hipMemcpyAsync(g_ss.x, xs + (size_t)b0 * w.cols, (size_t)m * w.cols * sizeof(float),
                                hipMemcpyHostToDevice, st));
-        int ks1 = 0;
-        if (m == 1 && w.dtype == DT_Q4T && q4t_kernel_m1x(w.kchunks, false, &ks1)) {
+        if (m == 1 && gemv_m1x_ok(w, g_ss.x)) {
             // one launch: the kernel stages its operand from the f32 row
             XSrc src{};
             src.mode = XS_ROWS;
@@ -779,6 +778,18 @@ int cmf_gemv_dev_noalloc(cmf_weight w, const float* d_x, int ldx, int b, float* 
     if (!base) return fail("gemv_dev_noalloc: no workspace on this device");
     float* xs = (float*)(base + NOALLOC_PLANES_MAX);
     hipStream_t st = stream();
+    if (b == 1 && gemv_m1x_ok(w->w, d_x)) {
+        // one launch: the kernel stages its operand from the f32 row (the
+        // same planes, so the same result bit for bit)
+        XSrc src{};
+        src.mode = XS_ROWS;
+        src.x = d_x;
+        src.ldx = w->w.cols;
+        const int rc = gemv(w->w, src, d_y, ldy, 1, 0, w->w.rows, false, st);
+        if (rc != CMF_OK) return rc;
+        CMF_HIP(hipGetLastError());
+        return CMF_OK;
+    }
     int rc = launch_prep(w->w, d_x, ldx, b, base, xs, st);
     if (rc != CMF_OK) return rc;
     rc = launch_gemv(w->w, base, xs, d_y, ldy, b, 0, w->w.rows, st);

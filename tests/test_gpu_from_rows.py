@@ -1,0 +1,61 @@
+"""GEMVs and FFNs from plain f32 rows: one-row GEMVs that stage their own
+operand (q8, q4t) equal the operand producer plus the prepared-operand GEMV
+bit for bit at every instance's step count, rows that no wide load fits keep
+the general producer, and the FFN of more than 16 rows (large-batch GEMMs)
+equals an f64 product."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(gpu, dt, rows, cols, seed=3):
+    from cmf_amd import synth
+    t = {"q8": synth.q8_uniform, "q4t": synth.q4t_uniform, "q4tp": synth.q4tp_uniform}[dt](seed, rows, cols)
+    return t, gpu.Weight(t["dtype"], rows, cols, payload=t["bytes"], q=t["q"], row_scale=t["row_scale"])
+
+
+# q8: the last column count of each instance (8, 16, 32, 64, 128, 192 steps of
+# 64), one step past it, a partial step, columns that are no multiple of 4
+Q8_COLS = [4, 100, 512, 516, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 12288, 12292, 1002]
+Q4_COLS = [32, 512, 544, 1024, 2048, 4096, 4128, 8192, 8224]
+
+
+@pytest.mark.parametrize("dt,cols", [("q8", c) for c in Q8_COLS] + [(d, c) for d in ("q4t", "q4tp") for c in Q4_COLS])
+def test_one_row_equals_prepared(gpu, dt, cols):
+    from cmf_amd import synth
+    rows, L = 37, gpu.lib()
+    t, w = _weight(gpu, dt, rows, cols)
+    pl, xs = gpu.DevBuf(L.cmf_prep_bytes(w.h)), gpu.DevBuf(256)
+    dx, dy = gpu.DevBuf((cols + 1) * 4), gpu.DevBuf(rows * 4)
+    wd = synth.dequant(t).astype(np.float64)
+    for x in (synth.normal(5, cols), np.zeros(cols, np.float32)):
+        for off in (0, 1):  # (an odd address: no wide loads)
+            buf = np.zeros(cols + 1, np.float32)
+            buf[off:off + cols] = x
+            dx.upload(buf)
+            gpu.check(L.cmf_prep_dev(w.h, dx.p + 4 * off, cols, 1, pl.p, xs.p))
+            gpu.check(L.cmf_gemv_prepared(w.h, pl.p, xs.p, 1, dy.p, rows, 0))
+            gpu.check(L.cmf_sync())
+            want = dy.download((rows,))
+            gpu.check(L.cmf_gemv_dev_noalloc(w.h, dx.p + 4 * off, cols, 1, dy.p, rows))
+            gpu.check(L.cmf_sync())
+            assert np.array_equal(dy.download((rows,)), want)
+            bound = 2.0 ** -22 * np.abs(x).max() * np.abs(wd).sum(1) + 2.0 ** -23 * (cols // 32 + 16) * (np.abs(wd) @ np.abs(x))
+            assert np.all(np.abs(want - wd @ x.astype(np.float64)) <= bound)
+    w.free()
+
+
+# batches of a split producer (items past a workgroup's 256, a partial one)
+@pytest.mark.parametrize("dt,cols,m", [("q4t", 2080, 13), ("q4tp", 4128, 9), ("q8", 4112, 16), ("q8", 1000, 6), ("q4t", 96, 2)])
+def test_batch_rows(gpu, dt, cols, m):
+    from cmf_amd import synth
+    rows = 53
+    t, w = _weight(gpu, dt, rows, cols, seed=9)
+    x = synth.normal(6, m * cols).reshape(m, cols)
+    got = gpu.matmul(w, x).astype(np.float64)
+    wd, xd = synth.dequant(t).astype(np.float64), x.astype(np.float64)
+    bound = (2.0 ** -22 * np.abs(xd).max(1)[:, None] * np.abs(wd).sum(1)[None, :]
+             + 2.0 ** -23 * (cols // 32 + 16) * (np.abs(xd) @ np.abs(wd).T))
+    assert np.all(np.abs(got - xd @ wd.T) <= bound)
+    w.free()
