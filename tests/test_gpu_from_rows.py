@@ -59,3 +59,30 @@ def test_batch_rows(gpu, dt, cols, m):
              + 2.0 ** -23 * (cols // 32 + 16) * (np.abs(xd) @ np.abs(wd).T))
     assert np.all(np.abs(got - xd @ wd.T) <= bound)
     w.free()
+
+
+@pytest.mark.parametrize("dt,hidden,inter,b", [("q4t", 256, 512, 17), ("q4tp", 288, 800, 65), ("q8", 320, 12320, 40),
+                                               ("q8", 90, 130, 33), ("q4t", 64, 96, 2100)])
+def test_ffn_large_batch(gpu, dt, hidden, inter, b):
+    from cmf_amd import synth
+    (t1, w1), (t3, w3), (t2, w2) = (_weight(gpu, dt, r, c, s) for r, c, s in
+                                    ((inter, hidden, 21), (inter, hidden, 22), (hidden, inter, 23)))
+    x = synth.normal(24, b * hidden).reshape(b, hidden) * np.float32(0.1)
+    out = np.empty((b, hidden), np.float32)
+    assert gpu.ffn(w1, w3, w2, x, b, hidden, inter, out)
+    d1, d3, d2 = (synth.dequant(t).astype(np.float64) for t in (t1, t3, t2))
+    g, u = x @ d1.T, x @ d3.T
+    h = g / (1 + np.exp(-g)) * u
+    ref = h @ d2.T
+    # three products of 22-bit operands and f32 sums, the first two through a
+    # SiLU of slope at most 1.1
+    eg, eu = (2.0 ** -22 * np.abs(x).max(1)[:, None] * np.abs(d).sum(1) + 2.0 ** -23 * (hidden // 32 + 16) * (np.abs(x) @ np.abs(d).T)
+              for d in (d1, d3))
+    eh = 1.1 * eg * np.abs(u) + np.abs(g) * eu + 2.0 ** -20 * np.abs(h)
+    bound = (eh @ np.abs(d2).T + 2.0 ** -22 * np.abs(h).max(1)[:, None] * np.abs(d2).sum(1)
+             + 2.0 ** -23 * (inter // 32 + 16) * (np.abs(h) @ np.abs(d2).T))
+    err = np.abs(out - ref)
+    print(f"{dt} {hidden}/{inter} b={b}: largest error / bound {np.max(err / bound):.3f}", flush=True)
+    assert np.all(err <= bound)
+    for w in (w1, w3, w2):
+        w.free()
