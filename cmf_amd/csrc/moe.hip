@@ -21,7 +21,10 @@
 //                     (k_moe_down_tok); caller-routed jobs: job j:
 //                     W_down[e_j] h, the operand made from the h rows in the
 //                     workgroup;
-//   other codecs or larger batches (grouped GEMVs over all b rows; rows of
+//   other codecs or larger batches (k_moe_rows, also over each job's own
+//   tokens, in passes of 5 or 8): 3. gate|up with the SwiGLU, 4. down with
+//   the operand made from the h rows in the workgroup;
+//   rows of more than 32 steps (grouped GEMVs over all b rows; rows of
 //   tokens that did not pick the expert are computed and ignored):
 //   3. gate|up, 3b. the per-job operand h = silu(g) * u, 4. down;
 //   5. k_moe_combine  out[t] = sum over ranks i of w[t][i] * down[job(t, i)][t],
@@ -582,6 +585,260 @@ __global__ __launch_bounds__(64 * RBW * KP, GU && KP > 1 ? 6 : 1) void k_moe_q4t
     }
 }
 
+// ---------------------------------------------------------------------------
+// Expert GEMVs over the job's own tokens for every codec and up to 16 tokens
+// (q4t at b <= 8 keeps k_moe_q4t): workgroups, LDS operand and split of a
+// row as there, in passes of at most SG token slots (q4: 8, the hi and lo
+// planes in A rows 0..7 and 8..15; q8: 5, the three planes in rows 5 p +
+// slot), each pass one MFMA per step and tile with the weights held in
+// registers from the first.  The grouped GEMVs this replaces multiplied all
+// b rows by every job's expert and read b operand rows per row block (48 KiB
+// at 16 rows of 1024 q8 columns, for 16 KiB of weights).  Bound by the weight
+// stream and latency.  Measured on MI355X, 64 q8 experts of 1024/512, top 8,
+// 16 tokens: gate|up 25.4 -> 14 us, down operand + down 22.7 -> 9.8.
+// ---------------------------------------------------------------------------
+template <int FMT, int RBW, int KP, int SPW, bool GU>
+__global__ __launch_bounds__(64 * RBW * KP) void k_moe_rows(MoeGx a) {
+    constexpr bool Q8 = FMT == DT_Q8ROW, TP = FMT == DT_Q4TP;
+    constexpr int NW = RBW * KP, NT = 64 * NW, SG = Q8 ? 5 : 8, NP = Q8 ? 3 : 2, C = Q8 ? 16 : 8;
+    extern __shared__ __align__(16) uint8_t smem[];  // operand [slot][item][plane] x 16 B, then (q4) tile biases [tile][16]
+    __shared__ float part[KP][RBW][16][17];          // (q8: int32 bits)
+    __shared__ float lad[TP ? NW : 1][TP ? 16 * 33 : 1];
+    __shared__ unsigned smax[SG];
+    __shared__ float sxs[SG];
+    const int j = blockIdx.y;
+    if (j >= a.jobs[0]) return;  // uniform
+    const GemvDesc d = a.desc[a.jobs[1 + j]];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, s = lane >> 4;
+    const int rbi = wave % RBW, kp = wave / RBW, g0 = kp * SPW;
+    const int nk = a.nk, M = a.M, rb = blockIdx.x * RBW + rbi, rbc = min(rb, a.nrb - 1);
+    const int* jl = a.jt + (size_t)j * MOE_JT;
+    const int n = min(jl[0], MAXB);
+    const int tokl = jl[1 + min(lane & 15, n - 1)];  // lane k (mod 16): the token of slot k
+    const float xsv = GU ? ldg(a.xs + (lane & 15)) : 0.f;
+    const int IT = nk * (Q8 ? 4 : 16), QI = IT * NP;
+    float* lb = (float*)(smem + (size_t)SG * QI * 16);
+    int4v wv[SPW];
+    uint2 sv[Q8 ? 1 : SPW];
+    auto load_weights = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < SPW; u++) {
+            const size_t t = (size_t)rbc * nk + min(g0 + u, nk - 1);
+            wv[u] = ld_stream((const int4v*)d.w + t * 64 + lane);
+            if constexpr (TP) sv[u].x = ldg((const uint32_t*)d.scale + t * 16 + r);
+            else if constexpr (!Q8) {
+                const uint64_t sw = ldg((const uint64_t*)d.scale + t * 16 + r);
+                sv[u] = make_uint2((uint32_t)sw, (uint32_t)(sw >> 32));
+            }
+        }
+    };
+    float rs = 0.f;
+    if constexpr (Q8) rs = ldg((const float*)d.scale + rbc * 16 + r);
+    if constexpr (TP) {
+        if (s == 0) {
+            const float2 p = ldg_f2(d.rowp + rbc * 16 + r);
+            float tv = p.x;
+            lad[wave][r * 33] = tv;
+            for (int c = 1; c < 32; c++) {
+                tv = tv * p.y;
+                lad[wave][r * 33 + c] = tv;
+            }
+        }
+    }
+    for (int p0 = 0; p0 < n; p0 += SG) {
+        const int ns = min(SG, n - p0);  // this pass's slots
+        if (p0 > 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the last pass has left the LDS
+        if constexpr (GU) {
+            // the slots' rows of the prepared planes, by direct loads
+            const int NI = ns * QI;
+            for (int c = wave; c * 64 < NI; c += NW) {
+                const int i = min(c * 64 + lane, NI - 1), slot = i / QI, rest = i - slot * QI;
+                const int pl = rest % NP, it = rest / NP, tok = __shfl(tokl, p0 + slot);
+                __builtin_amdgcn_global_load_lds((const void*)(a.planes + (((size_t)pl * IT + it) * M + tok) * 16),
+                                                 (__attribute__((address_space(3))) void*)(smem + c * 1024), 16, 0, 0);
+            }
+            if constexpr (!Q8) {
+                const float* T1 = (const float*)(a.planes + (size_t)2 * IT * M * 16);  // [tile][16] hi, then lo
+                const float* T2 = T1 + (size_t)nk * 4 * 16;
+                const int tokb = __shfl(tokl, p0 + min(lane & 7, ns - 1));
+                for (int c = wave; c < nk; c += NW)
+                    __builtin_amdgcn_global_load_lds((const void*)(((lane & 15) < 8 ? T1 : T2) + (size_t)(4 * c + s) * 16 + tokb),
+                                                     (__attribute__((address_space(3))) void*)(lb + c * 64), 4, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (p0 == 0) {
+                load_weights();
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vmcnt<(Q8 ? 1 : 2) * SPW>();  // the wave's share of the copy
+            } else {
+                wait_vmcnt<0>();
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else {
+            // the operand from the slots' f32 rows (the producer's planes and
+            // biases), C columns an item: their max |x| by LDS atomics first
+            const float* hx = a.hx + (size_t)j * a.hx_stride;
+            const int NI = ns * IT;
+            auto item = [&](int i, int& slot, int& it, float (&x)[C]) __attribute__((always_inline)) {
+                slot = i / IT;
+                it = i - slot * IT;
+                const int c0 = C * it, tok = __shfl(tokl, p0 + min(slot, ns - 1));
+                const bool in = i < NI && c0 < a.K;  // (K % 32 == 0: all inside or all past the row)
+                const float4v* src = (const float4v*)(hx + (size_t)tok * a.ldh + (in ? c0 : 0));
+#pragma unroll
+                for (int q = 0; q < C / 4; q++) {
+                    const float4v v = ldg(src + q);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[4 * q + e] = in ? v[e] : 0.f;
+                }
+            };
+            // (the first items stay in registers and are requested before the
+            // weights: a later load would wait for all of those)
+            int slot, it;
+            float x[C];
+            item(tid, slot, it, x);
+            __builtin_amdgcn_sched_barrier(0);
+            if (p0 == 0) load_weights();
+            __builtin_amdgcn_sched_barrier(0);
+            if (tid < SG) smax[tid] = 0u;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            for (int i0 = 0; i0 < NI; i0 += NT) {
+                if (i0 > 0) item(i0 + tid, slot, it, x);
+                float am = 0.f;
+#pragma unroll
+                for (int e = 0; e < C; e++) am = fmaxf(am, fabsf(x[e]));
+                if (i0 + tid < NI) atomicMax(&smax[slot], __float_as_uint(am));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            for (int i0 = 0; i0 < NI; i0 += NT) {  // (whole waves: the shuffles below)
+                if (NI > NT) item(i0 + tid, slot, it, x);
+                const bool on = i0 + tid < NI;
+                const float am = __uint_as_float(smax[on ? slot : 0]);
+                uint4* dst = (uint4*)smem + (on ? slot * QI + it * NP : 0);
+                if constexpr (Q8) {
+                    const float sx = am > 0.f ? am / 127.0f : 1.0f, inv = 1.0f / sx;
+                    uint32_t w0[4] = {}, w1[4] = {}, w2[4] = {};
+#pragma unroll
+                    for (int e = 0; e < 16; e++) q8_split(x[e], inv, e & 3, w0[e >> 2], w1[e >> 2], w2[e >> 2]);
+                    if (on) {
+                        dst[0] = make_uint4(w0[0], w0[1], w0[2], w0[3]);
+                        dst[1] = make_uint4(w1[0], w1[1], w1[2], w1[3]);
+                        dst[2] = make_uint4(w2[0], w2[1], w2[2], w2[3]);
+                        if (it == 0) sxs[slot] = sx;
+                    }
+                } else {
+                    float scale, xsl;
+                    q4_fix_scale(am, scale, xsl);
+                    constexpr int ord[8] = {0, 4, 2, 6, 1, 5, 3, 7};
+                    uint32_t hv[4] = {}, lv[4] = {};
+                    float sh = 0.f, sl = 0.f;  // (exact: integers and multiples of 2^-11)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        _Float16 h, l;
+                        q4_fix_split(x[ord[e]] * scale, h, l);
+                        hv[e >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, h) << (16 * (e & 1));
+                        lv[e >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, l) << (16 * (e & 1));
+                        sh += (float)h;
+                        sl += (float)l;
+                    }
+                    sh += __shfl_xor(sh, 1);
+                    sh += __shfl_xor(sh, 2);
+                    sl += __shfl_xor(sl, 1);
+                    sl += __shfl_xor(sl, 2);
+                    if (on) {
+                        dst[0] = make_uint4(hv[0], hv[1], hv[2], hv[3]);
+                        dst[1] = make_uint4(lv[0], lv[1], lv[2], lv[3]);
+                        if ((it & 3) == 0) {
+                            lb[(it >> 2) * 16 + slot] = sh * Q4_BIAS;
+                            lb[(it >> 2) * 16 + 8 + slot] = sl * Q4_BIAS;
+                        }
+                        if (it == 0) sxs[slot] = xsl;
+                    }
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        // A row r: plane pr of slot br (rows past the slots repeat one; their sums are not used)
+        const int pr = Q8 ? min(r / SG, 2) : r >> 3, br = min(Q8 ? r % SG : r & 7, ns - 1);
+        const int4v* X = (const int4v*)smem + br * QI + pr;
+        if constexpr (Q8) {
+            int4v acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < SPW; u++) {
+                const int4v z = {0, 0, 0, 0};
+                const int4v x = X[(min(g0 + u, nk - 1) * 4 + s) * NP];
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(g0 + u < nk ? x : z, wv[u], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) part[kp][rbi][4 * s + v][r] = __int_as_float(acc[v]);
+        } else {
+            float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < SPW; u++) {
+                const bool in = g0 + u < nk;  // (steps past the row: zero scale, a select)
+                const int uc = min(g0 + u, nk - 1);
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const half8 xa = __builtin_bit_cast(half8, X[((uc * 4 + t) * 4 + s) * NP]);
+                    const float4v cb = ((const float4v*)lb)[(uc * 4 + t) * 4 + s];  // A rows 4s..4s+3
+                    const float4v dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, dq_nib_word((uint32_t)wv[u][t]), cb, 0, 0, 0);
+                    float sc;
+                    if constexpr (TP) {
+                        sc = lad[wave][r * 33 + ((sv[u].x >> (5 * t)) & 31)];
+                    } else {
+                        const uint32_t sw = t < 2 ? sv[u].x : sv[u].y;
+                        sc = f16_bits_to_f32((t & 1) ? sw >> 16 : sw & 0xFFFFu);
+                    }
+                    if (!in) sc = 0.f;
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[v] += dd[v] * sc;
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) part[kp][rbi][4 * s + v][r] = acc[v];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (kp == 0) {  // the K parts' partials in part order; lane (r, s): weight row r of slots s, s + 4
+            float* y = a.y + (size_t)j * a.y_stride;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int b = s + 4 * q, bc = min(b, SG - 1);
+                float val;
+                const int tok = __shfl(tokl, p0 + min(b, ns - 1));
+                const float xsl = GU ? __shfl(xsv, tok) : sxs[min(b, ns - 1)];
+                if constexpr (Q8) {
+                    int t0 = 0, t1 = 0, t2 = 0;
+#pragma unroll
+                    for (int k = 0; k < KP; k++) {
+                        t0 += __float_as_int(part[k][rbi][bc][r]);
+                        t1 += __float_as_int(part[k][rbi][SG + bc][r]);
+                        t2 += __float_as_int(part[k][rbi][2 * SG + bc][r]);
+                    }
+                    val = (((float)t0 + (float)t1 * 0.0078125f + (float)t2 * 6.103515625e-05f) * xsl) * rs;
+                } else {
+                    float hi = 0.f, lo = 0.f;
+#pragma unroll
+                    for (int k = 0; k < KP; k++) {
+                        hi += part[k][rbi][bc][r];
+                        lo += part[k][rbi][8 + bc][r];
+                    }
+                    val = (hi + lo) * xsl * 16777216.0f;  // 2^24: denormal nibbles
+                }
+                if constexpr (GU) {
+                    const float u = __shfl_xor(val, 8);  // the matching up row
+                    const int row = 8 * rb + r;
+                    if (b < ns && r < 8 && rb < a.nrb && row < a.rows / 2)
+                        y[(size_t)tok * a.ldy + row] = (val / (1.0f + expf(-val))) * u;
+                } else {
+                    const int row = 16 * rb + r;
+                    if (b < ns && rb < a.nrb && row < a.rows) y[(size_t)tok * a.ldy + row] = val;
+                }
+            }
+        }
+    }
+}
+
 // Down projection and combine of routed batches in one launch (q4t, K =
 // inter <= 1024): workgroup (rb, t) computes rows [16 rb, 16 rb + 16) of
 // token t's MoE output; wave i (one per rank, k waves) multiplies expert
@@ -786,6 +1043,32 @@ MoeKernel moe_q4t_pick(int nk, bool gu, int* nw, int* rbw) {
     if (nk <= 16) return moe_q4t_inst<4, 2, 8>(gu, nw, rbw);
     return nullptr;
 }
+// k_moe_rows for rows of nk 1 KiB steps (nullptr: none); *nw = its waves,
+// *rbw its row blocks
+template <int FMT, int RBW, int KP, int SPW>
+MoeKernel moe_rows_inst(bool gu, int* nw, int* rbw) {
+    *nw = RBW * KP;
+    *rbw = RBW;
+    return gu ? k_moe_rows<FMT, RBW, KP, SPW, true> : k_moe_rows<FMT, RBW, KP, SPW, false>;
+}
+template <int FMT>
+MoeKernel moe_rows_by_nk(int nk, bool gu, int* nw, int* rbw) {
+    if (nk <= 4) return moe_rows_inst<FMT, 4, 1, 4>(gu, nw, rbw);
+    if (nk <= 8) return moe_rows_inst<FMT, 4, 1, 8>(gu, nw, rbw);
+    if (nk <= 12) return moe_rows_inst<FMT, 4, 2, 6>(gu, nw, rbw);
+    if (nk <= 16) return moe_rows_inst<FMT, 4, 2, 8>(gu, nw, rbw);
+    if (nk <= 32) return moe_rows_inst<FMT, 2, 4, 8>(gu, nw, rbw);
+    return nullptr;
+}
+MoeKernel moe_rows_pick(int dtype, int nk, bool gu, int* nw, int* rbw) {
+    return dtype == DT_Q8ROW ? moe_rows_by_nk<DT_Q8ROW>(nk, gu, nw, rbw)
+           : dtype == DT_Q4T ? moe_rows_by_nk<DT_Q4T>(nk, gu, nw, rbw)
+                             : moe_rows_by_nk<DT_Q4TP>(nk, gu, nw, rbw);
+}
+// its dynamic LDS: a pass's operand rows and (q4) the tile biases
+size_t moe_rows_lds(int dtype, int nk) {
+    return dtype == DT_Q8ROW ? (size_t)5 * nk * 4 * 3 * 16 : (size_t)8 * nk * 16 * 2 * 16 + (size_t)nk * 4 * 16 * 4;
+}
 }  // namespace cmf
 
 using namespace cmf;
@@ -905,6 +1188,41 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         d.rows = dw.rows;
         d.nrb = dw.rows_pad / 16;
         hipLaunchKernelGGL(kd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), ld, s, d);
+    } else if (MoeKernel xg = gather_env ? moe_rows_pick(gw.dtype, gw.kchunks, true, &sp1, &rw1) : nullptr,
+               xd = gather_env ? moe_rows_pick(dw.dtype, dw.kchunks, false, &sp2, &rw2) : nullptr;
+               xg && xd && moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks)) &&
+               moe_lds_ok(xd, moe_rows_lds(dw.dtype, dw.kchunks))) {
+        // the same two launches over each job's own tokens for any codec and
+        // up to 16 tokens
+        MoeGx g{};
+        g.desc = m->d_gu;
+        g.jobs = m->jobs;
+        g.jt = m->jt;
+        g.planes = m->px;
+        g.xs = m->xsx;
+        g.y = m->ygu;
+        g.y_stride = (size_t)MAXB * I;
+        g.ldy = I;
+        g.M = b;
+        g.nk = gw.kchunks;
+        g.rows = gw.rows;
+        g.nrb = gw.rows_pad / 16;
+        hipLaunchKernelGGL(xg, dim3((g.nrb + rw1 - 1) / rw1, mj), dim3(64 * sp1), moe_rows_lds(gw.dtype, gw.kchunks), s, g);
+        MoeGx d = g;
+        d.desc = m->d_down;
+        d.planes = nullptr;
+        d.xs = nullptr;
+        d.hx = m->ygu;
+        d.hx_stride = (size_t)MAXB * I;
+        d.ldh = I;
+        d.K = I;
+        d.y = m->yd;
+        d.y_stride = yd_stride;
+        d.ldy = H;
+        d.nk = dw.kchunks;
+        d.rows = dw.rows;
+        d.nrb = dw.rows_pad / 16;
+        hipLaunchKernelGGL(xd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), moe_rows_lds(dw.dtype, dw.kchunks), s, d);
     } else {
         rc = gemv_grouped(gw, m->d_gu, m->jobs, mj, m->px, 0, m->xsx, m->ygu, ygu_stride, 2 * I, b, s);
         if (rc != CMF_OK) return rc;
