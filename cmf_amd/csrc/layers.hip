@@ -248,10 +248,66 @@ __device__ __forceinline__ float2 attn_merge_row(const float* pm, const float* p
 // chunks of the output projection's q8 operand: x ~= cs (q0 + q1/128 +
 // q2/16384), cs = max|x| of the chunk / 127 (the layout and split of
 // prep8_row with one scale per chunk instead of per row).
-__global__ __launch_bounds__(64) void k_attn_merge(AttnArgs a) {
+// W > 1 (contexts of more than 32 chunks): the workgroup's wave w merges
+// chunks 32 w .. and the W sums meet in LDS, one memory round trip where one
+// wave walked 32 chunks at a time (12000 positions, 188 chunks: 9.8 -> 5.2 us).
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_attn_merge(AttnArgs a) {
     const int rh = blockIdx.x, b = rh / a.nh;
     const int used = (*a.pbase + a.padd + b + ATT_C) / ATT_C;
-    const float2 o = attn_merge_row<32>(a.pm, a.pl, a.po, a.nch, (size_t)rh, used, a.out + (size_t)rh * 128);
+    float2 o;
+    if constexpr (W == 1) {
+        o = attn_merge_row<32>(a.pm, a.pl, a.po, a.nch, (size_t)rh, used, a.out + (size_t)rh * 128);
+    } else {
+        __shared__ float sm[W], sl[W];
+        __shared__ float2 so[W][64];
+        const int wl = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        const size_t row = (size_t)rh * a.nch;
+        float M = -INFINITY, L = 0.f;
+        float2 O = make_float2(0.f, 0.f);
+        for (int c0 = 32 * wv; c0 < used; c0 += 32 * W) {
+            float2 ov[32];
+#pragma unroll
+            for (int j = 0; j < 32; j++) ov[j] = ((const float2*)a.po)[(row + min(c0 + j, used - 1)) * 64 + wl];
+            const int c = min(c0 + (wl & 31), used - 1);
+            const bool in = wl < 32 && c0 + wl < used;
+            const float mc = a.pm[row + c], lc = a.pl[row + c];
+            const float mx = fmaxf(M, wave_max(in ? mc : -INFINITY));
+            const float al = M == -INFINITY ? 0.f : expf(M - mx), w = in && mc != -INFINITY ? expf(mc - mx) : 0.f;
+            M = mx;
+            L = L * al + wave_sum(w * lc);
+            O.x *= al;
+            O.y *= al;
+#pragma unroll
+            for (int j = 0; j < 32; j++) {
+                const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+                O.x += wj * ov[j].x;
+                O.y += wj * ov[j].y;
+            }
+        }
+        if (wl == 0) {
+            sm[wv] = M;
+            sl[wv] = L;
+        }
+        so[wv][wl] = O;
+        __syncthreads();
+        if (wv) return;
+        float mx = sm[0];
+#pragma unroll
+        for (int w = 1; w < W; w++) mx = fmaxf(mx, sm[w]);
+        L = 0.f;
+        O = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const float f = sm[w] == -INFINITY ? 0.f : expf(sm[w] - mx);
+            L += sl[w] * f;
+            O.x += so[w][wl].x * f;
+            O.y += so[w][wl].y * f;
+        }
+        const float inv = L > 0.f ? 1.0f / L : 0.f;
+        o = make_float2(O.x * inv, O.y * inv);
+        ((float2*)(a.out + (size_t)rh * 128))[wl] = o;
+    }
     if (!a.wop) return;
     const int lane = threadIdx.x & 63, h = rh - b * a.nh, br = a.wop_b0 + b, nk = 2 * a.nh, M = a.wop_M;
     float am = fmaxf(fabsf(o.x), fabsf(o.y));
@@ -609,7 +665,10 @@ void launch_attention(const AttnArgs& a, int max_len, hipStream_t st, bool merge
     }
     hipLaunchKernelGGL(k, dim3(a.nkv, nch), dim3(256), 0, st, a);
     if (!a.attend || !merge) return;
-    hipLaunchKernelGGL(k_attn_merge, dim3(a.nb * a.nh), dim3(64), 0, st, a);
+    // (one wave holds 32 chunks at once)
+    if (nch <= 32) hipLaunchKernelGGL(k_attn_merge<1>, dim3(a.nb * a.nh), dim3(64), 0, st, a);
+    else if (nch <= 128) hipLaunchKernelGGL(k_attn_merge<4>, dim3(a.nb * a.nh), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(k_attn_merge<8>, dim3(a.nb * a.nh), dim3(512), 0, st, a);
 }
 
 int launch_argmax_part(const float* x, int ld, int n, int nrows, float* pv, int* pi, hipStream_t st) {

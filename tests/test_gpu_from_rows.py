@@ -86,3 +86,35 @@ def test_ffn_large_batch(gpu, dt, hidden, inter, b):
     assert np.all(err <= bound)
     for w in (w1, w3, w2):
         w.free()
+
+
+@pytest.mark.parametrize("pos", [2040, 2047, 2049, 4300, 8191, 8300])
+def test_long_context_merge(gpu, pos):
+    """attention over more than 32 chunks of 64 positions (several waves merge
+    them), against an f64 softmax over the exported keys and values"""
+    from cmf_amd import synth
+    from cmf_amd.model import Model
+    cfg = dict(n_layers=1, hidden=256, n_heads=2, n_kv=1, head_dim=128, inter=64, vocab=512, max_seq=8400, rope_theta=1e6, eps=1e-6)
+    sm = synth.synth_model(cfg, seed=43, norm_noise=0.1, sigma=0.05, mtp=False)
+    for n in ("gate", "up", "down"):
+        sm["layers"][0][n]["bytes"][:] = np.tile(np.array([0, 0] + [0x88] * 16, np.uint8), sm["layers"][0][n]["bytes"].size // 18)
+    m = Model(sm)
+    m.prefill(synth.ids(44, pos, 512))
+    tok = synth.ids(45, 1, 512)
+    hid, _ = m.forward_batch(tok, pos, want_logits=False)
+    k, v = (a[0].astype(np.float64) for a in m.kv_export(0, pos + 1))
+    m.free()
+    l, lm = sm["layers"][0], sm["lm_head"]
+    h = lm["q"][tok[0]].astype(np.float64) * lm["row_scale"][tok[0]]
+    rms = lambda x, w: x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-6) * w  # noqa: E731
+    q = rms((synth.dequant(l["wq"]).astype(np.float64) @ rms(h, l["input_norm"])).reshape(2, 128), l["q_norm"])
+    ang = (np.float32(pos) * (np.float32(1) / np.power(np.float32(1e6), np.arange(64, dtype=np.float32) / np.float32(64)))).astype(np.float64)
+    q = np.concatenate([q[:, :64] * np.cos(ang) - q[:, 64:] * np.sin(ang), q[:, :64] * np.sin(ang) + q[:, 64:] * np.cos(ang)], 1)
+    s = q @ k.T / np.sqrt(128.0)
+    p = np.exp(s - s.max(1, keepdims=True))
+    o = (p / p.sum(1, keepdims=True)) @ v
+    ref = h + synth.dequant(l["wo"]).astype(np.float64) @ o.reshape(-1)
+    err = np.linalg.norm(hid[0] - ref) / np.linalg.norm(ref)
+    print(f"position {pos}: {err:.1e}", flush=True)
+    # the angles' frequencies are one ulp from the host's: pos * 2^-24 in the scores
+    assert err < 1e-5 + pos * 2.0 ** -24
