@@ -97,10 +97,10 @@ GemvKernel q8_kernel(int m, int xm, int ks);
 // k_gemv_q4t_m1): the instance, its waves per workgroup (*ks) and dynamic
 // LDS bytes (*lds), or nullptr
 GemvKernel q8_kernel_m1(int nk, bool resid, int* ks, size_t* lds);
-GemvKernel q8_kernel_m1x(int nk, bool resid, int* ks);
+GemvKernel q8_kernel_m1x(int nk, int var, int* ks);
 GemvKernel q4t_kernel_m1(int nk, bool resid, int* ks, size_t* lds);
 // q4t, M = 1, the operand staged from its f32 row inside the kernel (XS_ROWS)
-GemvKernel q4t_kernel_m1x(int nk, bool resid, int* ks);
+GemvKernel q4t_kernel_m1x(int nk, int var, int* ks);
 
 enum { EPI_NONE = 0, EPI_SWIGLU = 1 };
 

@@ -643,7 +643,7 @@ bool gemv_m1x_ok(const DevWeight& w, const float* x) {
     s.ldx = w.cols;
     int ks = 0;
     if (!env || fused_lds_bytes(w, s, 1) == 0) return false;
-    return w.dtype == DT_Q4T ? w.cols % 8 == 0 && q4t_kernel_m1x(w.kchunks, false, &ks) : w.dtype == DT_Q8ROW && q8_kernel_m1x(w.kchunks, false, &ks);
+    return w.dtype == DT_Q4T ? w.cols % 8 == 0 && q4t_kernel_m1x(w.kchunks, M1X_ROWS, &ks) : w.dtype == DT_Q8ROW && q8_kernel_m1x(w.kchunks, M1X_ROWS, &ks);
 }
 
 constexpr int FUSED_MIN_KS = 8;  // waves of a workgroup that stages m > 2 rows
@@ -715,14 +715,20 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
             return CMF_OK;
         }
     }
-    // M = 1 from the f32 row (XS_ROWS; q4t, q8): the kernels that stage
-    // their own operand slices (CMF_GEMV_M1X=0 keeps the general fused kernel)
+    // M = 1 from the f32 row or its RMSNorm (q4t, q8): the kernels that
+    // stage their own operand slices (CMF_GEMV_M1X=0 keeps the general fused
+    // kernel).  A normed row of more than 1024 row blocks (the lm_head) keeps
+    // the general kernel, whose workgroups stage the row once for several
+    // blocks.  Measured on MI355X in the decode of a 2048-wide model: gate|up
+    // q4t 12288x2048 with SwiGLU 10.0 -> 6.5 us, qkv q8 4096x2048 6.3 -> 4.0.
     static const int m1x_env = env_int("CMF_GEMV_M1X", 1);
-    if (m1x_env && m == 1 && xm == XM_FUSED && a.src.mode == XS_ROWS && (w.dtype == DT_Q4T || w.dtype == DT_Q8ROW) &&
-        !grouped && grid_override <= 0 && ks_override <= 0 && a.epi == EPI_NONE &&
+    const bool m1_norm = a.src.mode == XS_NORM && a.nrb <= 1024 && !a.resid;
+    if (m1x_env && m == 1 && xm == XM_FUSED && (m1_norm || (a.src.mode == XS_ROWS && a.epi == EPI_NONE)) &&
+        (w.dtype == DT_Q4T || w.dtype == DT_Q8ROW) && !grouped && grid_override <= 0 && ks_override <= 0 &&
         (w.dtype == DT_Q8ROW || a.src.K % 8 == 0)) {
         int ks1 = 0;
-        GemvKernel k1 = w.dtype == DT_Q4T ? q4t_kernel_m1x(w.kchunks, a.resid, &ks1) : q8_kernel_m1x(w.kchunks, a.resid, &ks1);
+        const int var = m1_norm ? (a.epi == EPI_SWIGLU ? M1X_SWIGLU : M1X_NORM) : a.resid ? M1X_RESID : M1X_ROWS;
+        GemvKernel k1 = w.dtype == DT_Q4T ? q4t_kernel_m1x(w.kchunks, var, &ks1) : q8_kernel_m1x(w.kchunks, var, &ks1);
         if (k1 && resident_per_cu(k1, 64 * ks1, 0) >= 1) {
             void* args[] = {&a};
             CMF_HIP(hipLaunchKernel((const void*)k1, dim3(a.nrb), dim3(64 * ks1), args, 0, st));

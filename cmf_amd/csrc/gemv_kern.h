@@ -1049,6 +1049,47 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1(GemvArgs a) {
     }
 }
 
+// What the M = 1 kernels below make of their row: the plain row (+ the
+// residual epilogue), or the RMSNorm of it (+ the SwiGLU epilogue of a
+// gate|up weight, rows interleaved 8 / 8).
+enum { M1X_ROWS = 0, M1X_RESID = 1, M1X_NORM = 2, M1X_SWIGLU = 3 };
+// x <- rms_norm(x) * w on the lanes' pieces (inference.rs:33-50): the f64
+// sums of squares meet in LDS, one LDS-only barrier (the weights in flight)
+template <int KS, int NIT, int Q>
+__device__ __forceinline__ void m1x_norm(float4v (&xv)[NIT][Q], const float4v (&nv)[NIT][Q], const bool (&on)[NIT],
+                                         double* wss, int K, double eps, int wave, int lane) {
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < NIT; i++)
+#pragma unroll
+        for (int h = 0; h < Q; h++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) ss += on[i] ? (double)xv[i][h][k] * (double)xv[i][h][k] : 0.0;
+    ss = wave_sum(ss);
+    if (lane == 0) wss[wave] = ss;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    ss = wss[0];
+#pragma unroll
+    for (int w = 1; w < KS; w++) ss += wss[w];
+    const float inv = 1.0f / (float)sqrt(ss / (double)K + eps);
+#pragma unroll
+    for (int i = 0; i < NIT; i++)
+#pragma unroll
+        for (int h = 0; h < Q; h++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) xv[i][h][k] = xv[i][h][k] * inv * nv[i][h][k];
+}
+// the row's output (on: the lanes that hold rows r = 0 .. 15 of row block rb)
+template <bool RESID, bool SWI>
+__device__ __forceinline__ void m1x_store(const GemvArgs& a, float val, float yold, int row, int rb, int r, bool on) {
+    if constexpr (SWI) {
+        const float u = __shfl_xor(val, 8);  // the matching up row
+        if (on && r < 8 && rb < a.nrb) a.y[(a.rb0 + rb) * 8 + r] = (val / (1.0f + expf(-val))) * u;
+    } else if (on && row >= a.row_lo && row < a.row_hi && rb < a.nrb) {
+        a.y[row - a.row_lo] = RESID ? yold + val : val;
+    }
+}
+
 // q4t, M = 1, from the f32 operand row itself (XS_ROWS): the workgroup
 // needs no producer launch.  Wave w reads the SPW * 128 columns of its own
 // steps, one 8-column k-slot item per lane and step group, then the
@@ -1058,12 +1099,14 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1(GemvArgs a) {
 // would have written) into its own LDS region and runs the MFMA loop of
 // k_gemv_q4t_m1.  Columns past the row (steps past ntg, tiles past K) are
 // zero: their planes and biases vanish.
-template <int KS, int SPW, bool RESID>
+template <int KS, int SPW, int VAR>
 __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
+    constexpr bool RESID = VAR == M1X_RESID, NORM = VAR >= M1X_NORM, SWI = VAR == M1X_SWIGLU;
     constexpr int NIT = SPW / 4;           // 8-column items per lane (16 SPW items per wave)
     static_assert(SPW % 4 == 0 && SPW * 8 <= 64, "items per lane");
     __shared__ float part[KS][64];
     __shared__ float wmax[KS];
+    __shared__ double wss[NORM ? KS : 1];
     __shared__ __align__(16) uint4 slice[KS][SPW * 32];  // [item][plane] 16 B, item = (u * 4 + t) * 4 + s'
     __shared__ float sbias[KS][SPW * 8];                 // [(u * 4 + t) * 2 + plane]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1075,7 +1118,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
     const float yold = RESID ? ldg(a.y + (rowc - a.row_lo)) : 0.f;
     // this lane's items: item q = lane + 64 i = (u * 4 + t) * 4 + s', columns
     // 32 ((t0 + u) * 4 + t) + 8 s' .. + 7 (clamped loads, zero by select)
-    float4v xv[NIT][2];
+    float4v xv[NIT][2], nv[NORM ? NIT : 1][2];
     bool on[NIT];
 #pragma unroll
     for (int i = 0; i < NIT; i++) {
@@ -1085,6 +1128,11 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
         const float* src = a.src.x + (on[i] ? c0 : 0);
         xv[i][0] = ldg((const float4v*)src);
         xv[i][1] = ldg((const float4v*)(src + 4));
+        if constexpr (NORM) {
+            const float* wn = a.src.w + (on[i] ? c0 : 0);
+            nv[i][0] = ldg((const float4v*)wn);
+            nv[i][1] = ldg((const float4v*)(wn + 4));
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
     uint4 wv[SPW];
@@ -1099,6 +1147,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
     wait_vmcnt<2 * SPW>();  // this wave's operand columns are in
+    if constexpr (NORM) m1x_norm<KS, NIT, 2>(xv, nv, on, wss, K, a.src.eps, wave, lane);
     float am = 0.f;
 #pragma unroll
     for (int i = 0; i < NIT; i++)
@@ -1170,10 +1219,8 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
     }
     float o = m1_reduce<KS>(part, acc, wave, lane);
     o += __shfl_xor(o, 32);  // hi rows (lanes s = 0, 1) + lo rows (s = 2, 3)
-    if (wave == 0 && s == 0 && row >= a.row_lo && row < a.row_hi && rb < a.nrb) {
-        const float val = o * xs * 16777216.0f;  // 2^24: denormal nibbles
-        a.y[row - a.row_lo] = RESID ? yold + val : val;
-    }
+    const float val = o * xs * 16777216.0f;  // 2^24: denormal nibbles
+    m1x_store<RESID, SWI>(a, val, yold, row, rb, r, wave == 0 && s == 0);
 }
 
 // q8, M = 1, from the f32 operand row itself (XS_ROWS), as k_gemv_q4t_m1x:
@@ -1184,11 +1231,13 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q4t_m1x(GemvArgs a) {
 // k_gemv_q8_m1, whose per-wave sums are exact: equal to producer +
 // k_gemv_q8_m1 bit for bit.  Latency-bound: 1024x1024 producer launch + GEMV
 // 6.4 us a call, this 3.7.  K % 4 == 0; columns past K are zero.
-template <int KS, int SPW, bool RESID>
+template <int KS, int SPW, int VAR>
 __global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
+    constexpr bool RESID = VAR == M1X_RESID, NORM = VAR >= M1X_NORM, SWI = VAR == M1X_SWIGLU;
     constexpr int NIT = (SPW * 16 + 63) / 64;  // 4-column pieces per lane
     __shared__ float part[KS][64];
     __shared__ float wmax[KS];
+    __shared__ double wss[NORM ? KS : 1];
     // item i = (u * 4 + s') * 3 + p: plane p of step u, k-slot s'
     __shared__ __align__(16) uint32_t slice[KS][SPW * 4 * 3 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1198,13 +1247,14 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
     const int rowc = max(a.row_lo, min(row, a.row_hi - 1));
     const float rs = ldg((const float*)a.scale + row);
     const float yold = RESID ? ldg(a.y + (rowc - a.row_lo)) : 0.f;
-    float4v xv[NIT];
+    float4v xv[NIT][1], nv[NORM ? NIT : 1][1];
     bool on[NIT];
 #pragma unroll
     for (int i = 0; i < NIT; i++) {
         const int q = lane + 64 * i, c = c0 * 64 + 4 * q;
         on[i] = q < SPW * 16 && c < K;
-        xv[i] = ldg((const float4v*)(a.src.x + (on[i] ? c : 0)));
+        xv[i][0] = ldg((const float4v*)(a.src.x + (on[i] ? c : 0)));
+        if constexpr (NORM) nv[i][0] = ldg((const float4v*)(a.src.w + (on[i] ? c : 0)));
     }
     __builtin_amdgcn_sched_barrier(0);
     int4v wv[SPW];
@@ -1213,11 +1263,12 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
     for (int u = 0; u < SPW; u++) wv[u] = ldg((const int4v*)a.w + (wbase + min(c0 + u, nkc - 1)) * 64 + lane);
     __builtin_amdgcn_sched_barrier(0);
     wait_vmcnt<SPW>();  // this wave's operand columns are in
+    if constexpr (NORM) m1x_norm<KS, NIT, 1>(xv, nv, on, wss, K, a.src.eps, wave, lane);
     float am = 0.f;
 #pragma unroll
     for (int i = 0; i < NIT; i++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) am = fmaxf(am, on[i] ? fabsf(xv[i][k]) : 0.f);
+        for (int k = 0; k < 4; k++) am = fmaxf(am, on[i] ? fabsf(xv[i][0][k]) : 0.f);
     am = wave_max(am);
     if (lane == 0) wmax[wave] = am;
     // LDS-only barrier: the weights stay in flight
@@ -1232,7 +1283,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
         const int q = lane + 64 * i;
         uint32_t b0 = 0, b1 = 0, b2 = 0;
 #pragma unroll
-        for (int k = 0; k < 4; k++) q8_split(on[i] ? xv[i][k] : 0.f, inv, k, b0, b1, b2);
+        for (int k = 0; k < 4; k++) q8_split(on[i] ? xv[i][0][k] : 0.f, inv, k, b0, b1, b2);
         if (q < SPW * 16) {
             uint32_t* d = slice[wave] + (q >> 2) * 12 + (q & 3);
             d[0] = b0;
@@ -1254,10 +1305,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemv_q8_m1x(GemvArgs a) {
     }
     const float v = (float)acc[0] + (float)acc[1] * 0.0078125f + (float)acc[2] * 6.103515625e-05f;
     const float o = m1_reduce<KS>(part, v, wave, lane);
-    if (wave == 0 && s == 0 && row >= a.row_lo && row < a.row_hi && rb < a.nrb) {
-        const float val = (o * xs) * rs;
-        a.y[row - a.row_lo] = RESID ? yold + val : val;
-    }
+    m1x_store<RESID, SWI>(a, (o * xs) * rs, yold, row, rb, r, wave == 0 && s == 0);
 }
 
 // Instance of the M = 1 kernels for rows of nk 1 KiB steps (nullptr: none);
@@ -1289,32 +1337,36 @@ inline GemvKernel q8_m1_pick(int nk, bool resid, int* ks, size_t* lds) {
     return nullptr;
 }
 template <int KS, int SPW>
-inline GemvKernel q8_m1x_inst(bool resid, int* ks) {
+inline GemvKernel q8_m1x_inst(int var, int* ks) {
     *ks = KS;
-    return resid ? k_gemv_q8_m1x<KS, SPW, true> : k_gemv_q8_m1x<KS, SPW, false>;
+    return var == M1X_ROWS ? k_gemv_q8_m1x<KS, SPW, M1X_ROWS>
+           : var == M1X_RESID ? k_gemv_q8_m1x<KS, SPW, M1X_RESID>
+           : var == M1X_NORM ? k_gemv_q8_m1x<KS, SPW, M1X_NORM> : k_gemv_q8_m1x<KS, SPW, M1X_SWIGLU>;
 }
 // (the waves and steps of q8_m1_pick, so that the sums are the same)
-inline GemvKernel q8_m1x_pick(int nk, bool resid, int* ks) {
-    if (nk <= 8) return q8_m1x_inst<1, 8>(resid, ks);
-    if (nk <= 16) return q8_m1x_inst<8, 2>(resid, ks);
-    if (nk <= 32) return q8_m1x_inst<8, 4>(resid, ks);
-    if (nk <= 64) return q8_m1x_inst<16, 4>(resid, ks);
-    if (nk <= 128) return q8_m1x_inst<16, 8>(resid, ks);
-    if (nk <= 192) return q8_m1x_inst<16, 12>(resid, ks);
+inline GemvKernel q8_m1x_pick(int nk, int var, int* ks) {
+    if (nk <= 8) return q8_m1x_inst<1, 8>(var, ks);
+    if (nk <= 16) return q8_m1x_inst<8, 2>(var, ks);
+    if (nk <= 32) return q8_m1x_inst<8, 4>(var, ks);
+    if (nk <= 64) return q8_m1x_inst<16, 4>(var, ks);
+    if (nk <= 128) return q8_m1x_inst<16, 8>(var, ks);
+    if (nk <= 192) return q8_m1x_inst<16, 12>(var, ks);
     return nullptr;
 }
 template <int KS, int SPW>
-inline GemvKernel q4t_m1x_inst(bool resid, int* ks) {
+inline GemvKernel q4t_m1x_inst(int var, int* ks) {
     *ks = KS;
-    return resid ? k_gemv_q4t_m1x<KS, SPW, true> : k_gemv_q4t_m1x<KS, SPW, false>;
+    return var == M1X_ROWS ? k_gemv_q4t_m1x<KS, SPW, M1X_ROWS>
+           : var == M1X_RESID ? k_gemv_q4t_m1x<KS, SPW, M1X_RESID>
+           : var == M1X_NORM ? k_gemv_q4t_m1x<KS, SPW, M1X_NORM> : k_gemv_q4t_m1x<KS, SPW, M1X_SWIGLU>;
 }
 // the staged-from-rows kernel: SPW a multiple of 4 (whole items per lane)
-inline GemvKernel q4t_m1x_pick(int nk, bool resid, int* ks) {
-    if (nk <= 4) return q4t_m1x_inst<1, 4>(resid, ks);
-    if (nk <= 8) return q4t_m1x_inst<2, 4>(resid, ks);
-    if (nk <= 16) return q4t_m1x_inst<4, 4>(resid, ks);
-    if (nk <= 32) return q4t_m1x_inst<8, 4>(resid, ks);
-    if (nk <= 64) return q4t_m1x_inst<8, 8>(resid, ks);
+inline GemvKernel q4t_m1x_pick(int nk, int var, int* ks) {
+    if (nk <= 4) return q4t_m1x_inst<1, 4>(var, ks);
+    if (nk <= 8) return q4t_m1x_inst<2, 4>(var, ks);
+    if (nk <= 16) return q4t_m1x_inst<4, 4>(var, ks);
+    if (nk <= 32) return q4t_m1x_inst<8, 4>(var, ks);
+    if (nk <= 64) return q4t_m1x_inst<8, 8>(var, ks);
     return nullptr;  // (16 waves x 8 steps of slices would pass the 64 KiB of static LDS)
 }
 inline GemvKernel q4t_m1_pick(int nk, bool resid, int* ks, size_t* lds) {

@@ -88,6 +88,28 @@ def test_ffn_large_batch(gpu, dt, hidden, inter, b):
         w.free()
 
 
+@pytest.mark.parametrize("attn,ffn,H,I,n", [("q8", "q4t", 256, 512, 9), ("q8", "q8", 320, 608, 5), ("q4t", "q4t", 1056, 544, 5),
+                                            ("q8", "q4t", 2048, 6144, 3)])
+def test_one_row_blocks_equal_batches(gpu, attn, ffn, H, I, n):
+    """one-row decoder blocks (the norm and the SwiGLU inside the one-row
+    GEMVs) leave the rows that batches of rows (the general kernels) leave"""
+    from cmf_amd import DT_Q4T, DT_Q8ROW, synth
+    from cmf_amd.model import Model
+    cfg = dict(n_layers=2, hidden=H, n_heads=2, n_kv=1, head_dim=128, inter=I, vocab=512, max_seq=64, rope_theta=1e6, eps=1e-6)
+    dt = {"q8": DT_Q8ROW, "q4t": DT_Q4T}
+    m = Model(synth.synth_model(cfg, seed=41, norm_noise=0.1, sigma=0.05, mtp=False, attn_dtype=dt[attn], ffn_dtype=dt[ffn]))
+    ids = synth.ids(42, n, 512)
+    rows = np.concatenate([m.forward_batch(ids[p:p + 1], p, want_logits=False)[0] for p in range(n)])
+    both, lg = m.forward_batch(ids, 0)
+    one = m.forward_batch(ids[n - 1:], n - 1)[1]
+    err = np.linalg.norm(rows - both) / np.linalg.norm(both)
+    print(f"{attn}/{ffn} {H}/{I}: rows {err:.1e}", flush=True)
+    # seven products of 22-bit operands and f32 sums a layer (5e-7 each)
+    assert err < 1e-5
+    assert np.linalg.norm(one[0] - lg[-1]) < 1e-5 * np.linalg.norm(lg[-1])
+    m.free()
+
+
 @pytest.mark.parametrize("pos", [2040, 2047, 2049, 4300, 8191, 8300])
 def test_long_context_merge(gpu, pos):
     """attention over more than 32 chunks of 64 positions (several waves merge
