@@ -691,7 +691,16 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
         xm = XM_PREPC;
     } else if (a.src.mode == XS_GLOBAL) {
         lds = lds_bytes(w, m);
-        if (lds > LDSX_MAX) lds = 0;  // planes read in place from global memory
+        // planes read in place from global memory: past the LDS budget, or
+        // where the kernel's static LDS leaves them no room on a CU (q8, 16
+        // rows of 2561..2730 columns)
+        if (lds > LDSX_MAX) lds = 0;
+        if (lds) {
+            GemvKernel kp = w.dtype == DT_Q8ROW ? q8_kernel(m, XM_PREP, ks)
+                            : w.dtype == DT_Q4T ? q4t_kernel(m, XM_PREP, ks, 1)
+                                                : q4tp_kernel(m, XM_PREP, ks, 1);
+            if (!kp || resident_per_cu(kp, 64 * ks, lds) < 1) lds = 0;
+        }
         xm = lds ? XM_PREP : XM_GLOBAL;
     } else {
         lds = fused_lds_bytes(w, a.src, m);

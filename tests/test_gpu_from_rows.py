@@ -140,3 +140,15 @@ def test_long_context_merge(gpu, pos):
     print(f"position {pos}: {err:.1e}", flush=True)
     # the angles' frequencies are one ulp from the host's: pos * 2^-24 in the scores
     assert err < 1e-5 + pos * 2.0 ** -24
+
+
+@pytest.mark.parametrize("cols", [2560, 2592, 2720, 2752])
+def test_operand_at_the_lds_limit(gpu, cols):
+    """16 q8 rows whose planes just fit, do not fit beside the kernel's static
+    LDS, and are past the budget"""
+    from cmf_amd import synth
+    t, w = _weight(gpu, "q8", 40, cols)
+    x = synth.normal(8, 16 * cols).reshape(16, cols)
+    got, ref = gpu.matmul(w, x).astype(np.float64), x.astype(np.float64) @ synth.dequant(t).astype(np.float64).T
+    assert np.linalg.norm(got - ref) < 2e-6 * np.linalg.norm(ref)
+    w.free()
