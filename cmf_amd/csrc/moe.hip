@@ -618,7 +618,8 @@ __global__ __launch_bounds__(64 * RBW * KP) void k_moe_rows(MoeGx a) {
     const int tokl = jl[1 + min(lane & 15, n - 1)];  // lane k (mod 16): the token of slot k
     const float xsv = GU ? ldg(a.xs + (lane & 15)) : 0.f;
     const int IT = nk * (Q8 ? 4 : 16), QI = IT * NP;
-    float* lb = (float*)(smem + (size_t)SG * QI * 16);
+    const int PS = min(SG, a.ns);  // slots a pass
+    float* lb = (float*)(smem + (size_t)PS * QI * 16);
     int4v wv[SPW];
     uint2 sv[Q8 ? 1 : SPW];
     auto load_weights = [&]() __attribute__((always_inline)) {
@@ -646,8 +647,8 @@ __global__ __launch_bounds__(64 * RBW * KP) void k_moe_rows(MoeGx a) {
             }
         }
     }
-    for (int p0 = 0; p0 < n; p0 += SG) {
-        const int ns = min(SG, n - p0);  // this pass's slots
+    for (int p0 = 0; p0 < n; p0 += PS) {
+        const int ns = min(PS, n - p0);  // this pass's slots
         if (p0 > 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the last pass has left the LDS
         if constexpr (GU) {
             // the slots' rows of the prepared planes, by direct loads
@@ -1065,9 +1066,9 @@ MoeKernel moe_rows_pick(int dtype, int nk, bool gu, int* nw, int* rbw) {
            : dtype == DT_Q4T ? moe_rows_by_nk<DT_Q4T>(nk, gu, nw, rbw)
                              : moe_rows_by_nk<DT_Q4TP>(nk, gu, nw, rbw);
 }
-// its dynamic LDS: a pass's operand rows and (q4) the tile biases
-size_t moe_rows_lds(int dtype, int nk) {
-    return dtype == DT_Q8ROW ? (size_t)5 * nk * 4 * 3 * 16 : (size_t)8 * nk * 16 * 2 * 16 + (size_t)nk * 4 * 16 * 4;
+// its dynamic LDS: the operand rows of a pass of ps slots and (q4) the tile biases
+size_t moe_rows_lds(int dtype, int nk, int ps) {
+    return dtype == DT_Q8ROW ? (size_t)ps * nk * 4 * 3 * 16 : (size_t)ps * nk * 16 * 2 * 16 + (size_t)nk * 4 * 16 * 4;
 }
 }  // namespace cmf
 
@@ -1190,10 +1191,13 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         hipLaunchKernelGGL(kd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), ld, s, d);
     } else if (MoeKernel xg = gather_env ? moe_rows_pick(gw.dtype, gw.kchunks, true, &sp1, &rw1) : nullptr,
                xd = gather_env ? moe_rows_pick(dw.dtype, dw.kchunks, false, &sp2, &rw2) : nullptr;
-               xg && xd && moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks)) &&
-               moe_lds_ok(xd, moe_rows_lds(dw.dtype, dw.kchunks))) {
+               xg && xd && moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks, 8)) &&
+               moe_lds_ok(xd, moe_rows_lds(dw.dtype, dw.kchunks, 8))) {
         // the same two launches over each job's own tokens for any codec and
-        // up to 16 tokens
+        // up to 16 tokens; a pass holds twice the tokens that an expert gets
+        // on average (fewer slots of LDS leave room for more workgroups; a
+        // busier job takes another pass)
+        const int ps = std::min(std::min(8, b), std::max(2, (2 * b * k + m->ne - 1) / m->ne));
         MoeGx g{};
         g.desc = m->d_gu;
         g.jobs = m->jobs;
@@ -1207,7 +1211,8 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         g.nk = gw.kchunks;
         g.rows = gw.rows;
         g.nrb = gw.rows_pad / 16;
-        hipLaunchKernelGGL(xg, dim3((g.nrb + rw1 - 1) / rw1, mj), dim3(64 * sp1), moe_rows_lds(gw.dtype, gw.kchunks), s, g);
+        g.ns = ps;
+        hipLaunchKernelGGL(xg, dim3((g.nrb + rw1 - 1) / rw1, mj), dim3(64 * sp1), moe_rows_lds(gw.dtype, gw.kchunks, ps), s, g);
         MoeGx d = g;
         d.desc = m->d_down;
         d.planes = nullptr;
@@ -1222,7 +1227,7 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         d.nk = dw.kchunks;
         d.rows = dw.rows;
         d.nrb = dw.rows_pad / 16;
-        hipLaunchKernelGGL(xd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), moe_rows_lds(dw.dtype, dw.kchunks), s, d);
+        hipLaunchKernelGGL(xd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), moe_rows_lds(dw.dtype, dw.kchunks, ps), s, d);
     } else {
         rc = gemv_grouped(gw, m->d_gu, m->jobs, mj, m->px, 0, m->xsx, m->ygu, ygu_stride, 2 * I, b, s);
         if (rc != CMF_OK) return rc;
