@@ -1177,12 +1177,18 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
     DState hs{};
     int np = m->next_pos_host;
     int r0 = 0;
-    if (spec && m->use_graph && n > 1) {
+    // (a single round or step replays the captured one if there is one, but
+    // does not pay for a capture)
+    auto valid = [&](bool have, int sampling_was, int len, int need) {
+        return have && sampling_was == (int)sampling && len >= need;
+    };
+    if (spec && m->use_graph && n > 0) {
         // The captured round reads every position-dependent value from the
         // device state; only the attention grid is sized on the host, by a
         // bound on the positions these n rounds can reach (512-position steps).
         const int need = std::min(m->c.max_seq, ((np + (n + 1) * (k + 1) + 511) / 512) * 512);
-        if (!m->round_graph || m->graph_k != k || m->graph_sampling != (int)sampling || m->graph_len < need) {
+        const bool ok = m->graph_k == k && valid(m->round_graph, m->graph_sampling, m->graph_len, need);
+        if (!ok && n > 1) {
             // one eager round first: it sets the kernels' launch attributes
             spec_round(m, k, sampling, m->sc, np, s);
             r0 = 1;
@@ -1201,14 +1207,17 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
             m->graph_sampling = (int)sampling;
             m->graph_len = need;
         }
-        for (int r = r0; r < n; r++) CMF_HIP(hipGraphLaunch(m->round_graph, s));
-        r0 = n;
+        if (ok || n > 1) {
+            for (int r = r0; r < n; r++) CMF_HIP(hipGraphLaunch(m->round_graph, s));
+            r0 = n;
+        }
     }
-    if (!spec && m->use_graph && n > 1) {
+    if (!spec && m->use_graph && n > 0) {
         // plain steps the same way: one eager step, then one captured step
         // replayed (the forward_token_graph counterpart, gpu.rs:1368)
         const int need = std::min(m->c.max_seq, ((np + n + 2 + 511) / 512) * 512);
-        if (!m->plain_graph || m->plain_sampling != (int)sampling || m->plain_len < need) {
+        const bool ok = valid(m->plain_graph, m->plain_sampling, m->plain_len, need);
+        if (!ok && n > 1) {
             plain_step(m, sampling, m->sc, np, s);
             np += 1;
             r0 = 1;
@@ -1226,8 +1235,10 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
             m->plain_sampling = (int)sampling;
             m->plain_len = need;
         }
-        for (int r = r0; r < n; r++) CMF_HIP(hipGraphLaunch(m->plain_graph, s));
-        r0 = n;
+        if (ok || n > 1) {
+            for (int r = r0; r < n; r++) CMF_HIP(hipGraphLaunch(m->plain_graph, s));
+            r0 = n;
+        }
     }
     for (int r = r0; r < n; r++) {
         if (spec) {
@@ -1402,8 +1413,17 @@ int cmf_decode(cmf_model m, int max_tokens, const cmf_sampler_config* sc, uint64
         if (spec == 2) mon_token(mon, generated, wall_ms());
         const bool off = spec == 2 && (mon.phase == CMF_SPEC_PLAIN_TRIAL || mon.phase == CMF_SPEC_OFF);
         const bool sp = spec && !off && generated + 2 < max_tokens;
+        // Every round that the loop is sure to run whatever its drafts do
+        // (at most k + 1 tokens a round; plain steps one each) in one call,
+        // which replays a captured round without a host round trip between
+        // them; rounds under the monitor are timed one by one.  Where the
+        // positions would not fit, one at a time up to the same error.
+        const int per = sp ? k + 1 : 1, left = max_tokens - generated;
+        int n = spec == 2 ? 1 : sp ? (left - 2 + k) / (k + 1) : left - 1;
+        if (spec && !sp) n = 1;
+        n = std::max(1, std::min(n, (m->c.max_seq - 2 - m->next_pos_host) / per - 1));
         const double t0 = wall_ms();
-        rc = cmf_decode_rounds(m, 1, sp ? 1 : 0, k, &st);
+        rc = cmf_decode_rounds(m, n, sp ? 1 : 0, k, &st);
         if (rc != CMF_OK) return rc;
         ms += st.device_ms;
         tot.drafted += st.drafted;
@@ -1412,14 +1432,14 @@ int cmf_decode(cmf_model m, int max_tokens, const cmf_sampler_config* sc, uint64
         const int produced = m->emitted_host - generated;
         generated = m->emitted_host;
         if (sp) {
-            mon.spec_rounds += 1;
+            mon.spec_rounds += n;
             if (spec == 2) {
                 const double now = wall_ms();
                 mon_round(mon, now - t0, produced);
                 mon_after_round(mon, generated, now);
             }
         } else {
-            mon.plain_steps += 1;
+            mon.plain_steps += n;
         }
     }
     const int n = cmf_decode_tokens(m, out, m->emitted_host);
