@@ -146,6 +146,8 @@ struct cmf_model_s {
     float* pf_rlog = nullptr;
     size_t pf_rlog_cap = 0;
     _Float16* pf_khl = nullptr;  // the prefill attention's K / V operands (f16 hi / lo keys, then f32 values)
+    void* pf_part = nullptr;                 // the prefill attention's halves of long query blocks
+    unsigned long long* pf_mcell = nullptr;  // and the tags by which they meet
     unsigned long long* pf_cells = nullptr;  // placement check of the XCD prefill attention
     int* pf_err = nullptr;
     unsigned long long pf_tag = 0;
@@ -577,10 +579,16 @@ static int prefill_chunk() {
 }
 
 int ensure_prefill_bufs(cmf_model_s* m) {
-    if (m->pf_h) return CMF_OK;
+    if (m->pf_err) return CMF_OK;  // (the last of them)
     const auto& c = m->c;
     const int H = c.hidden, QKV = (c.n_heads + 2 * c.n_kv) * c.head_dim;
     const size_t R = std::min(prefill_chunk(), c.max_seq);
+    if (prefill_attention_fits(c.n_heads, c.n_kv, c.head_dim)) {
+        const size_t cells = prefill_attention_cells((int)R, c.n_heads, c.n_kv);
+        if (dalloc(m, &m->pf_part, prefill_attention_scratch((int)R, c.n_heads, c.n_kv)) || dalloc_t(m, &m->pf_mcell, cells))
+            return CMF_ERR;
+        CMF_HIP(hipMemset(m->pf_mcell, 0, cells * sizeof(unsigned long long)));
+    }
     if (dalloc_t(m, &m->pf_h, R * H) || dalloc_t(m, &m->pf_qkv, R * QKV) ||
         dalloc_t(m, &m->pf_ao, R * c.n_heads * c.head_dim) || dalloc_t(m, &m->pf_gu, R * 2 * c.inter) ||
         dalloc_t(m, &m->pf_hm, R * H) || dalloc_t(m, &m->pf_toks, R) ||
@@ -630,7 +638,7 @@ void prefill_attention(cmf_model_s* m, LayerDev& l, const float* qkv, float* ao,
         // the whole chunk at once: the tiled prefill attention (one launch
         // for the norms + append, one for the attention)
         PrefillAttnArgs pa{qkv, QKV, l.q_norm, l.k_norm, m->rope, l.kc, l.vc, c.max_seq, cnt, p0, nh, nkv,
-                           c.eps, m->pf_q, attend ? ao : nullptr, m->pf_khl, m->pf_cells, m->pf_err, ++m->pf_tag,
+                           c.eps, m->pf_q, attend ? ao : nullptr, m->pf_khl, m->pf_part, m->pf_mcell, m->pf_cells, m->pf_err, ++m->pf_tag,
                            !m->pf_xcd_off};
         launch_prefill_attention(pa, s);
         return;

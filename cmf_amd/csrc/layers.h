@@ -58,7 +58,9 @@ void launch_attention(const AttnArgs& a, int max_len, hipStream_t st, bool merge
 // rows' K / V appended to the cache, out [cnt][nh * 128] (out == nullptr:
 // only the append).  qbuf: [cnt][nh][128] scratch for the rotated queries;
 // khl: scratch for the rearranged K / V operands, nkv * npad * 128 * 8 bytes
-// (npad = ceil((p0 + cnt) / 128) * 128).
+// (npad = ceil((p0 + cnt) / 128) * 128).  part, mcell: where the two halves of
+// a long query block's keys meet (prefill_attention_scratch bytes;
+// prefill_attention_cells tags, zeroed once, for tags that never repeat).
 struct PrefillAttnArgs {
     const float* qkv;
     int ldq;
@@ -70,6 +72,8 @@ struct PrefillAttnArgs {
     float* qbuf;
     float* out;
     _Float16* khl;
+    void* part;
+    unsigned long long* mcell;
     // placement check of the XCD variant (kv head from the XCD a workgroup
     // runs on): cells [query block][8] take the launch's tag, a collision
     // sets *perr; cells == nullptr or !allow_xcd: the grid-indexed variant
@@ -78,8 +82,10 @@ struct PrefillAttnArgs {
     unsigned long long tag;
     bool allow_xcd;
 };
-constexpr int PREFILL_XCD_CELLS = 8 * 1024;  // query blocks of a chunk x 8 kv heads (2048 rows at 2 per block)
+constexpr int PREFILL_XCD_CELLS = 8 * 1024;  // workgroups of a kv head x 8 kv heads
 bool prefill_attention_fits(int nh, int nkv, int hd);
+size_t prefill_attention_cells(int cnt, int nh, int nkv);
+size_t prefill_attention_scratch(int cnt, int nh, int nkv);
 int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st);
 // The lexicographic (value, index) maximum step of argmax (sampler.rs:1130-1154
 // keeps the higher index on equal values; NaN never wins).
