@@ -95,6 +95,8 @@ __global__ __launch_bounds__(512) void k_prep_gemm(XSrc s, int K, int nitems, ui
             v[i][4 * q + 2] = in ? x.z : 0.f;
             v[i][4 * q + 3] = in ? x.w : 0.f;
         }
+        // (192 columns a lane: fewer loads in flight, or two registers spill)
+        if constexpr (MODE == XS_SILU && NI * C > 128) if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (MODE == XS_NORM) {
         double ss = 0.0;

@@ -402,8 +402,10 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
         }
         if (!run && split) {  // (uniform per workgroup) the other unit has the other half of these rows' keys
             const size_t cell = (size_t)pi * nkv + g;
-            float4v* mine = pt + (2 * cell + upper) * (FQ * HD / 4) + wave * 512 + lane;
-            float2v* ml = pml + 2 * cell * 256 + wave * 64 + lane;  // (both halves' waves hold them)
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // (these addresses are not worth registers across the tiles)
+            float4v* mine = pt + (2 * cell + upper) * (FQ * HD / 4) + wave * 512 + ln;
+            float2v* ml = pml + 2 * cell * 256 + wave * 64 + ln;  // (both halves' waves hold them)
             const auto seen = [&](bool first) {
                 if (t == 0) {
                     s_second = (first ? __hip_atomic_load(mcell + cell, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)
@@ -421,8 +423,8 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
                 second = seen(false);
                 if (!second) continue;
             }
-            const float4v* its = pt + (2 * cell + (upper ^ 1)) * (FQ * HD / 4) + wave * 512 + lane;
-            const float2v iml = pml[(2 * cell + (upper ^ 1)) * 256 + rg * 64 + lane];
+            const float4v* its = pt + (2 * cell + (upper ^ 1)) * (FQ * HD / 4) + wave * 512 + ln;
+            const float2v iml = pml[(2 * cell + (upper ^ 1)) * 256 + rg * 64 + ln];
             const float own = M;
             M = fmaxf(M, iml[0]);
             fm = weight(own);
