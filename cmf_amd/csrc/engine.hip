@@ -1080,10 +1080,10 @@ int cmf_prefill(cmf_model m, const int32_t* ids, int n) {
 int cmf_model_prefill_xcd(cmf_model m) { return m ? (m->pf_xcd_off ? 0 : 1) : CMF_ERR; }
 
 // logits of the tip hidden -> next token (greedy argmax or device sampler)
-static void pick_from_tip(cmf_model m, bool sampling, const cmf_sampler_config* sc, hipStream_t s) {
+static void pick_from_tip(cmf_model m, bool sampling, hipStream_t s) {
     const int H = m->c.hidden;
     gemv_f(m, m->lm, src_norm(m->h_tip, H, m->final_norm, m->c.eps), m->logits, m->c.vocab, 1, false, s);
-    if (sampling) sample_rows(m->sb, m->logits, m->c.vocab, 1, *sc, m->st, SampleMode::Plain, 0, nullptr, s);
+    if (sampling) sample_rows(m->sb, m->logits, m->c.vocab, 1, nullptr, m->st, SampleMode::Plain, 0, nullptr, s);
     else launch_argmax(m->logits, m->c.vocab, m->c.vocab, 1, m->am_v, m->am_i, m->st->argmax, s);
 }
 
@@ -1091,8 +1091,7 @@ static void pick_from_tip(cmf_model m, bool sampling, const cmf_sampler_config* 
 // device state: K chained MTP drafts, the K+1-row verify, acceptance, the
 // MTP re-warm of the verified pairs and the commit.  np = next_pos (host
 // mirror, sizes the attention grids).
-static void spec_round(cmf_model m, int k, bool sampling, const cmf_sampler_config& sc, int np,
-                       hipStream_t s, int graph_len = 0) {
+static void spec_round(cmf_model m, int k, bool sampling, int np, hipStream_t s, int graph_len = 0) {
     const int H = m->c.hidden, V = m->c.vocab;
     int* pb = &m->st->next_pos;
     for (int j = 0; j < k; j++) {
@@ -1100,13 +1099,13 @@ static void spec_round(cmf_model m, int k, bool sampling, const cmf_sampler_conf
         float* bufs[2] = {m->hm, m->hm2};
         const float* hin = j == 0 ? m->h_tip : bufs[(j - 1) & 1];
         mtp_step(m, tok, hin, bufs[j & 1], pb, j - 1, graph_len ? graph_len : np + j, s);
-        if (sampling) sample_rows(m->sb, m->logits, V, 1, sc, m->st, SampleMode::Draft, j, nullptr, s);
+        if (sampling) sample_rows(m->sb, m->logits, V, 1, nullptr, m->st, SampleMode::Draft, j, nullptr, s);
         else launch_argmax(m->logits, V, V, 1, m->am_v, m->am_i, &m->st->drafts[j], s);
     }
     launch_embed(m->st->drafts, embed_src(m), H, m->hv, H, k + 1, s, &m->st->t_next);
     trunk_forward(m, k + 1, pb, 0, graph_len ? graph_len : np + k + 1, true, s);
     if (sampling) {
-        sample_rows(m->sb, m->logits, V, k + 1, sc, m->st, SampleMode::Accept, k, m->out, s);
+        sample_rows(m->sb, m->logits, V, k + 1, nullptr, m->st, SampleMode::Accept, k, m->out, s);
     } else {
         const int ns = launch_argmax_part(m->logits, V, V, k + 1, m->am_v, m->am_i, s);
         hipLaunchKernelGGL(k_argmax_accept, dim3(1), dim3(64 * (k + 1)), 0, s, m->am_v, m->am_i, ns, m->st, k,
@@ -1119,13 +1118,12 @@ static void spec_round(cmf_model m, int k, bool sampling, const cmf_sampler_conf
 // One plain decode step: forward t_next at next_pos, emit it, pick the next.
 // graph_len > 0: the attention length bound of a captured step (every
 // position-dependent value is read from the device state).
-static void plain_step(cmf_model m, bool sampling, const cmf_sampler_config& sc, int np, hipStream_t s,
-                       int graph_len = 0) {
+static void plain_step(cmf_model m, bool sampling, int np, hipStream_t s, int graph_len = 0) {
     const int H = m->c.hidden, V = m->c.vocab;
     int* pb = &m->st->next_pos;
     launch_embed(&m->st->t_next, embed_src(m), H, m->hv, H, 1, s);
     trunk_forward(m, 1, pb, 0, graph_len ? graph_len : np + 1, true, s);
-    if (sampling) sample_rows(m->sb, m->logits, V, 1, sc, m->st, SampleMode::Plain, 0, nullptr, s);
+    if (sampling) sample_rows(m->sb, m->logits, V, 1, nullptr, m->st, SampleMode::Plain, 0, nullptr, s);
     else launch_argmax(m->logits, V, V, 1, m->am_v, m->am_i, m->st->argmax, s);
     hipLaunchKernelGGL(k_plain_commit, dim3(1), dim3(256), 0, s, m->st, m->hv, m->h_tip, H, m->out,
                        sampling ? 1 : 0);
@@ -1152,11 +1150,12 @@ int cmf_decode_begin(cmf_model m, const cmf_sampler_config* sc, uint64_t seed) {
     init.next_pos = m->next_pos_host;
     init.rng = seed;
     init.forced = -1;
+    init.samp = samp_cfg(*sc, m->c.vocab);
     CMF_HIP(hipMemcpyAsync(m->st, &init, sizeof(DState), hipMemcpyHostToDevice, s));
     CMF_HIP(hipStreamSynchronize(s));
     m->sc = *sc;
     const bool sampling = sc->temperature >= 1e-6f;
-    pick_from_tip(m, sampling, sc, s);
+    pick_from_tip(m, sampling, s);
     hipLaunchKernelGGL(k_first_token, dim3(1), dim3(1), 0, s, m->st, sampling ? 1 : 0);
     CMF_HIP(hipStreamSynchronize(s));
     CMF_HIP(hipGetLastError());
@@ -1198,7 +1197,7 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
         const bool ok = m->graph_k == k && valid(m->round_graph, m->graph_sampling, m->graph_len, need);
         if (!ok && n > 1) {
             // one eager round first: it sets the kernels' launch attributes
-            spec_round(m, k, sampling, m->sc, np, s);
+            spec_round(m, k, sampling, np, s);
             r0 = 1;
             if (m->round_graph) {
                 (void)hipGraphExecDestroy(m->round_graph);
@@ -1206,7 +1205,7 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
             }
             hipGraph_t g;
             CMF_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            spec_round(m, k, sampling, m->sc, np, s, need);
+            spec_round(m, k, sampling, np, s, need);
             CMF_HIP(hipStreamEndCapture(s, &g));
             const hipError_t ie = hipGraphInstantiate(&m->round_graph, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -1226,7 +1225,7 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
         const int need = std::min(m->c.max_seq, ((np + n + 2 + 511) / 512) * 512);
         const bool ok = valid(m->plain_graph, m->plain_sampling, m->plain_len, need);
         if (!ok && n > 1) {
-            plain_step(m, sampling, m->sc, np, s);
+            plain_step(m, sampling, np, s);
             np += 1;
             r0 = 1;
             if (m->plain_graph) {
@@ -1235,7 +1234,7 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
             }
             hipGraph_t g;
             CMF_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            plain_step(m, sampling, m->sc, np, s, need);
+            plain_step(m, sampling, np, s, need);
             CMF_HIP(hipStreamEndCapture(s, &g));
             const hipError_t ie = hipGraphInstantiate(&m->plain_graph, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -1250,12 +1249,12 @@ static int decode_rounds_impl(cmf_model m, int n, int spec, int k, cmf_gen_stats
     }
     for (int r = r0; r < n; r++) {
         if (spec) {
-            spec_round(m, k, sampling, m->sc, np, s);
+            spec_round(m, k, sampling, np, s);
             CMF_HIP(hipMemcpyAsync(&hs, m->st, sizeof(DState), hipMemcpyDeviceToHost, s));
             CMF_HIP(hipStreamSynchronize(s));
             np = hs.next_pos;
         } else {
-            plain_step(m, sampling, m->sc, np, s);
+            plain_step(m, sampling, np, s);
             np += 1;
         }
     }
@@ -1544,7 +1543,7 @@ static int verify_step_impl(cmf_model m, const int32_t* tokens, int b, int pos0,
     launch_embed(m->st->drafts, embed_src(m), H, m->hv, H, b, s, &m->st->t_next);
     trunk_forward(m, b, pb, 0, pos0 + b, true, s);
     if (sampling) {
-        sample_rows(m->sb, m->logits, V, b, *sc, m->st, SampleMode::Accept, k, m->out, s, b);
+        sample_rows(m->sb, m->logits, V, b, sc, m->st, SampleMode::Accept, k, m->out, s, b);
         if (argmax_out) launch_argmax(m->logits, V, V, b, m->am_v, m->am_i, m->st->argmax, s);
     } else {
         const int ns = launch_argmax_part(m->logits, V, V, b, m->am_v, m->am_i, s);

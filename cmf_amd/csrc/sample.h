@@ -16,8 +16,17 @@ constexpr int SPARSE_CAP = 4 * SPARSE_K_MAX + 64;
 static_assert(SPARSE_CAP % 64 == 0, "candidate lists are whole waves");
 constexpr int SLICE = 4096;       // logits per selection block
 
-// Decode state kept in HBM; kernels read positions from it so a round needs
-// no host values.
+// The sampling chain's settings as the kernels take them.
+struct SampCfg {
+    float t;      // temperature
+    float top_p;
+    float min_p;
+    int k;        // top_k, at most the vocabulary
+};
+SampCfg samp_cfg(const cmf_sampler_config& sc, int V);
+
+// Decode state kept in HBM; kernels read positions and the sampler's settings
+// from it so a round needs no host values.
 struct DState {
     int next_pos;        // next trunk position (trunk KV holds [0, next_pos))
     int a;               // accepted drafts of the last round
@@ -30,6 +39,7 @@ struct DState {
     unsigned long long rng;  // SplitMix64 state (sampler.rs:54-84)
     int drafts[16];
     int argmax[17];
+    SampCfg samp;            // the settings of this decode
 };
 
 enum class SampleMode { Draft, Plain, Accept };
@@ -61,8 +71,10 @@ int sample_alloc(SampleBufs& b, int V, const std::function<int(void**, size_t)>&
 //   Accept: rows 0..k against q_0..q_{k-1}; emits [t_next, accepted drafts]
 //           into out, sets a, forced, t_new (correction or draw from row a)
 // nuni > 0: the chain's uniforms are b.uni[0..nuni) in order (the caller's
-// shared uniforms), then the SplitMix64 stream.
-void sample_rows(SampleBufs& b, const float* logits, int V, int rows, const cmf_sampler_config& sc,
+// shared uniforms), then the SplitMix64 stream.  sc == nullptr: the settings
+// are st->samp, read by the kernels, so that a captured round serves every
+// sampler.
+void sample_rows(SampleBufs& b, const float* logits, int V, int rows, const cmf_sampler_config* sc,
                  DState* st, SampleMode mode, int j_or_k, int* out, hipStream_t s, int nuni = 0);
 
 // The sparse distribution of logits row 0 (sparse_distribution_into with the

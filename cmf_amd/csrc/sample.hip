@@ -25,11 +25,6 @@
 
 namespace cmf {
 
-struct SampCfg {
-    float t, top_p, min_p;
-    int k;
-};
-
 __device__ __forceinline__ uint32_t fkey(float f) {
     const uint32_t u = __float_as_uint(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
@@ -272,10 +267,11 @@ __device__ void select_topk_reg(const float (&v)[NPT], const int (&id)[NPT], int
 }
 
 __global__ __launch_bounds__(256) void k_topk_slice(const float* __restrict__ logits, int V, SampCfg c,
-                                                    int nslices, int* __restrict__ cid,
+                                                    const SampCfg* cp, int nslices, int* __restrict__ cid,
                                                     float* __restrict__ cv, float* __restrict__ smax,
                                                     float* __restrict__ ssum, int* __restrict__ ocnt,
                                                     int* __restrict__ oid) {
+    if (cp) c = *cp;
     const int sl = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
     __shared__ int hist[16][257];  // copies 257 apart: one bucket's copies fall in distinct banks
     __shared__ __align__(16) float tv[SPARSE_K_MAX + 256];
@@ -368,7 +364,7 @@ __global__ __launch_bounds__(256) void k_topk_slice(const float* __restrict__ lo
     }
 }
 
-__global__ __launch_bounds__(256) void k_topk_merge(int V, SampCfg c, int nslices,
+__global__ __launch_bounds__(256) void k_topk_merge(int V, SampCfg c, const SampCfg* cp, int nslices,
                                                     const int* __restrict__ cid,
                                                     const float* __restrict__ cv,
                                                     const float* __restrict__ smax,
@@ -376,6 +372,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(int V, SampCfg c, int nslice
                                                     const int* __restrict__ oid, int* __restrict__ rid,
                                                     float* __restrict__ rv, int* __restrict__ rn,
                                                     float* __restrict__ lmax, float* __restrict__ sum) {
+    if (cp) c = *cp;
     const int row = blockIdx.x, t = threadIdx.x;
     __shared__ int hist[16][257];  // copies 257 apart: one bucket's copies fall in distinct banks
     __shared__ __align__(16) float tv[SPARSE_K_MAX + 256];
@@ -847,13 +844,14 @@ __device__ void wload(WList& l, const int* ids, const float* ps, int n) {
     }
 }
 
-__global__ __launch_bounds__(64) void k_sample_finish(SampCfg c, int mode, int jk, const int* __restrict__ rid,
+__global__ __launch_bounds__(64) void k_sample_finish(SampCfg c, const SampCfg* cp, int mode, int jk, const int* __restrict__ rid,
                                                       const float* __restrict__ rv, const int* __restrict__ rn,
                                                       const float* __restrict__ lmax,
                                                       const float* __restrict__ sum, int* __restrict__ qid,
                                                       float* __restrict__ qp, int* __restrict__ qn, DState* st,
                                                       int* __restrict__ out, const float* __restrict__ uni,
                                                       int nuni) {
+    if (cp) c = *cp;
     const int lane = threadIdx.x;
     Uni rng{st->rng, uni, nuni, 0};
     if (mode == 0 || mode == 1) {  // Draft / Plain: distribution of row 0, one draw
@@ -981,7 +979,7 @@ int sample_alloc(SampleBufs& b, int V, const std::function<int(void**, size_t)>&
     return CMF_OK;
 }
 
-static SampCfg samp_cfg(const cmf_sampler_config& sc, int V) {
+SampCfg samp_cfg(const cmf_sampler_config& sc, int V) {
     SampCfg c;
     c.t = sc.temperature > 0.f ? sc.temperature : 1.0f;
     c.top_p = sc.top_p;
@@ -993,22 +991,23 @@ static SampCfg samp_cfg(const cmf_sampler_config& sc, int V) {
 void sample_distribution(SampleBufs& b, const float* logits, int V, const cmf_sampler_config& sc, int* ids,
                          float* probs, int* n, hipStream_t s) {
     const SampCfg c = samp_cfg(sc, V);
-    hipLaunchKernelGGL(k_topk_slice, dim3(b.nslices, 1), dim3(256), 0, s, logits, V, c, b.nslices, b.cid, b.cv,
+    hipLaunchKernelGGL(k_topk_slice, dim3(b.nslices, 1), dim3(256), 0, s, logits, V, c, nullptr, b.nslices, b.cid, b.cv,
                        b.smax, b.ssum, b.ocnt, b.oid);
-    hipLaunchKernelGGL(k_topk_merge, dim3(1), dim3(256), 0, s, V, c, b.nslices, b.cid, b.cv, b.smax, b.ssum,
+    hipLaunchKernelGGL(k_topk_merge, dim3(1), dim3(256), 0, s, V, c, nullptr, b.nslices, b.cid, b.cv, b.smax, b.ssum,
                        b.ocnt, b.oid, b.rid, b.rv, b.rn, b.lmax, b.sum);
     hipLaunchKernelGGL(k_sample_dist, dim3(1), dim3(64), 0, s, c, b.rid, b.rv, b.rn, b.lmax, b.sum, ids, probs, n);
 }
 
-void sample_rows(SampleBufs& b, const float* logits, int V, int rows, const cmf_sampler_config& sc,
+void sample_rows(SampleBufs& b, const float* logits, int V, int rows, const cmf_sampler_config* sc,
                  DState* st, SampleMode mode, int jk, int* out, hipStream_t s, int nuni) {
-    const SampCfg c = samp_cfg(sc, V);
-    hipLaunchKernelGGL(k_topk_slice, dim3(b.nslices, rows), dim3(256), 0, s, logits, V, c, b.nslices, b.cid,
+    const SampCfg c = sc ? samp_cfg(*sc, V) : SampCfg{};
+    const SampCfg* cp = sc ? nullptr : &st->samp;
+    hipLaunchKernelGGL(k_topk_slice, dim3(b.nslices, rows), dim3(256), 0, s, logits, V, c, cp, b.nslices, b.cid,
                        b.cv, b.smax, b.ssum, b.ocnt, b.oid);
-    hipLaunchKernelGGL(k_topk_merge, dim3(rows), dim3(256), 0, s, V, c, b.nslices, b.cid, b.cv, b.smax,
+    hipLaunchKernelGGL(k_topk_merge, dim3(rows), dim3(256), 0, s, V, c, cp, b.nslices, b.cid, b.cv, b.smax,
                        b.ssum, b.ocnt, b.oid, b.rid, b.rv, b.rn, b.lmax, b.sum);
     const int m = mode == SampleMode::Draft ? 0 : (mode == SampleMode::Plain ? 1 : 2);
-    hipLaunchKernelGGL(k_sample_finish, dim3(1), dim3(64), 0, s, c, m, jk, b.rid, b.rv, b.rn, b.lmax, b.sum, b.qid,
+    hipLaunchKernelGGL(k_sample_finish, dim3(1), dim3(64), 0, s, c, cp, m, jk, b.rid, b.rv, b.rn, b.lmax, b.sum, b.qid,
                        b.qp, b.qn, st, out, b.uni, nuni);
 }
 

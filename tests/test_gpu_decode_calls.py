@@ -1,0 +1,40 @@
+"""Decode calls one after another on one model: each takes its own sampler,
+whatever rounds an earlier call left captured."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CFG = dict(n_layers=2, hidden=256, n_heads=4, n_kv=2, head_dim=128, inter=512, vocab=4096, max_seq=256, rope_theta=1e6,
+           eps=1e-6)
+
+
+@pytest.fixture(scope="module")
+def calls(gpu):
+    from cmf_amd import synth
+    return synth.synth_model(CFG, seed=5, norm_noise=0.1, sigma=0.05), synth.ids(19, 20, CFG["vocab"])
+
+
+def _decode(m, prompt, *args, **kw):
+    m.prefill(prompt)
+    return m.decode(*args, **kw)[0].tolist()
+
+
+# (auto: five speculative rounds, then the last token, whatever the monitor measures)
+@pytest.mark.parametrize("spec,n,k", [(False, 16, 4), (True, 24, 3), ("auto", 6, 1)])
+def test_each_call_uses_its_sampler(gpu, calls, spec, n, k):
+    from cmf_amd import SamplerConfig
+    from cmf_amd.model import Model
+    sm, prompt = calls
+    samplers = [SamplerConfig(0.8, 0.9, 1, 1.0, 0.05), SamplerConfig(1.5, 1.0, 64, 1.0, 0.0), SamplerConfig(1.5, 0.3, 64, 1.0, 0.0)]
+    fresh = []
+    for s in samplers:
+        m = Model(sm)
+        fresh.append(_decode(m, prompt, n, sampler=s, seed=77, spec=spec, k=k))
+        m.free()
+    assert len({tuple(f) for f in fresh}) == len(fresh)
+    m = Model(sm)
+    for s, want in list(zip(samplers, fresh)) + [(samplers[0], fresh[0])]:
+        if spec == "auto":  # (rounds under the monitor replay what a decode of several rounds has captured)
+            _decode(m, prompt, 24, sampler=samplers[0], seed=3, spec=True, k=k)
+        assert _decode(m, prompt, n, sampler=s, seed=77, spec=spec, k=k) == want
+    m.free()
