@@ -1425,9 +1425,15 @@ int cmf_decode(cmf_model m, int max_tokens, const cmf_sampler_config* sc, uint64
         // which replays a captured round without a host round trip between
         // them; rounds under the monitor are timed one by one.  Where the
         // positions would not fit, one at a time up to the same error.
-        const int per = sp ? k + 1 : 1, left = max_tokens - generated;
-        int n = spec == 2 ? 1 : sp ? (left - 2 + k) / (k + 1) : left - 1;
-        if (spec && !sp) n = 1;
+        // (a k out of range is left to be refused by the round)
+        const int left = max_tokens - generated;
+        int n = 1, per = 1;
+        if (sp && spec == 1 && k >= 1 && k <= 8) {
+            per = k + 1;
+            n = (left - 2 + k) / per;
+        } else if (!spec) {
+            n = left - 1;
+        }
         n = std::max(1, std::min(n, (m->c.max_seq - 2 - m->next_pos_host) / per - 1));
         const double t0 = wall_ms();
         rc = cmf_decode_rounds(m, n, sp ? 1 : 0, k, &st);

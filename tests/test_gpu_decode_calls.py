@@ -1,5 +1,6 @@
-"""Decode calls one after another on one model: each takes its own sampler,
-whatever rounds an earlier call left captured."""
+"""Decode calls: a refused draft count, and calls one after another on one
+model, where each takes its own sampler, whatever rounds an earlier call left
+captured."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -37,4 +38,18 @@ def test_each_call_uses_its_sampler(gpu, calls, spec, n, k):
         if spec == "auto":  # (rounds under the monitor replay what a decode of several rounds has captured)
             _decode(m, prompt, 24, sampler=samplers[0], seed=3, spec=True, k=k)
         assert _decode(m, prompt, n, sampler=s, seed=77, spec=spec, k=k) == want
+    m.free()
+
+
+@pytest.mark.parametrize("k", [-1, 0, 9])
+def test_bad_draft_count_is_refused(gpu, calls, k):
+    from cmf_amd import CmfError
+    from cmf_amd.model import Model
+    sm, prompt = calls
+    m = Model(sm)
+    m.prefill(prompt)
+    for spec in (True, "auto"):
+        with pytest.raises(CmfError, match="k must be 1..8"):
+            m.decode(12, spec=spec, k=k)
+    assert len(m.decode(12, spec=False, k=k)[0]) == 12  # (plain steps take no drafts)
     m.free()
