@@ -358,6 +358,10 @@ __global__ __launch_bounds__(256) void k_moe_combine_rows(const float* __restric
 //       workgroup, exactly as the producer would prepare them, and
 //       y[t][16 rb + r] = the row's dot product.
 // ---------------------------------------------------------------------------
+// LDS bytes of an operand of ns slots of items 16-byte items: whole 1 KiB
+// chunks, as the direct loads fill it (the last chunk's lanes past the operand
+// repeat an item there; what follows must not be under them).
+__host__ __device__ constexpr size_t moe_opnd_lds(int ns, int items) { return ((size_t)ns * items * 16 + 1023) & ~(size_t)1023; }
 struct MoeGx {
     const GemvDesc* desc;
     const int* jobs;
@@ -366,7 +370,7 @@ struct MoeGx {
     const float* xs;        // GU: xs[t] of the operand
     float* y;         // + j * y_stride, token t's row at t * ldy
     size_t y_stride;
-    int ldy, M, nk, nrb, rows, ns;  // ns: token slots of the LDS copy (>= any job's count)
+    int ldy, M, nk, nrb, rows, ns;  // ns: token slots of the LDS operand (k_moe_q4t: >= any job's count; k_moe_rows: of a pass)
     // !GU: the operand rows themselves, f32: token t of job j at hx + j * hx_stride + t * ldh, K columns
     const float* hx;
     size_t hx_stride;
@@ -400,7 +404,7 @@ __global__ __launch_bounds__(64 * RBW * KP, GU && KP > 1 ? 6 : 1) void k_moe_q4t
 #pragma unroll
     for (int k = 1; k < 8; k++) tokv = ls == k ? tk[k] : tokv;
     const int QI = ntg * 32;  // items of one slot: (step, tile, k-slot) x plane
-    float* lb = (float*)(smem + (size_t)a.ns * QI * 16);
+    float* lb = (float*)(smem + moe_opnd_lds(a.ns, QI));
     uint4 wv[SPW];
     uint2 sv[SPW];
     // the weights + tile scales of the wave's row block (clamped: every load unconditional)
@@ -619,7 +623,7 @@ __global__ __launch_bounds__(64 * RBW * KP) void k_moe_rows(MoeGx a) {
     const float xsv = GU ? ldg(a.xs + (lane & 15)) : 0.f;
     const int IT = nk * (Q8 ? 4 : 16), QI = IT * NP;
     const int PS = min(SG, a.ns);  // slots a pass
-    float* lb = (float*)(smem + (size_t)PS * QI * 16);
+    float* lb = (float*)(smem + moe_opnd_lds(PS, QI));
     int4v wv[SPW];
     uint2 sv[Q8 ? 1 : SPW];
     auto load_weights = [&]() __attribute__((always_inline)) {
@@ -1068,7 +1072,7 @@ MoeKernel moe_rows_pick(int dtype, int nk, bool gu, int* nw, int* rbw) {
 }
 // its dynamic LDS: the operand rows of a pass of ps slots and (q4) the tile biases
 size_t moe_rows_lds(int dtype, int nk, int ps) {
-    return dtype == DT_Q8ROW ? (size_t)ps * nk * 4 * 3 * 16 : (size_t)ps * nk * 16 * 2 * 16 + (size_t)nk * 4 * 16 * 4;
+    return dtype == DT_Q8ROW ? moe_opnd_lds(ps, nk * 12) : moe_opnd_lds(ps, nk * 32) + (size_t)nk * 4 * 16 * 4;
 }
 }  // namespace cmf
 
@@ -1141,7 +1145,7 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         kd = moe_q4t_pick(dw.kchunks, false, &sp2, &rw2);
     }
     // LDS: the operand rows of up to b tokens + the tile biases
-    const size_t lg = (size_t)gw.kchunks * (b * 512 + 256), ld = (size_t)dw.kchunks * (b * 512 + 256);
+    const size_t lg = moe_rows_lds(DT_Q4T, gw.kchunks, b), ld = moe_rows_lds(DT_Q4T, dw.kchunks, b);
     if (kg && kd && moe_lds_ok(kg, lg) && moe_lds_ok(kd, ld)) {
         // gate|up -> h = silu(g) * u [job][t][I] (in the ygu area), then
         // down over the listed h rows -> yd [job][t][H]
