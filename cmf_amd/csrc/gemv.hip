@@ -561,9 +561,12 @@ int launch_prep(const DevWeight& w, const float* x, int ldx, int m, uint8_t* pla
 }
 
 static size_t lds_bytes(const DevWeight& w, int m) {
-    // q4: hi + lo planes and the tile biases [tile][16] f32 (m > 8: both tables)
-    return w.dtype == DT_Q8ROW ? (size_t)w.kchunks * 64 * 3 * m
-                               : (size_t)w.kchunks * 4 * (128 * m + (m > 8 ? 128 : 64));
+    // q4: hi + lo planes and the tile biases [tile][16] f32 (m > 8: both
+    // tables); whole 1 KiB chunks, as the copy fills them (the lanes of the
+    // last chunk past the operand repeat an item)
+    const size_t n = w.dtype == DT_Q8ROW ? (size_t)w.kchunks * 64 * 3 * m
+                                         : (size_t)w.kchunks * 4 * (128 * m + (m > 8 ? 128 : 64));
+    return (n + 1023) & ~(size_t)1023;
 }
 // LDS of a GEMV that evaluates the producer of src itself (XM_FUSED): the
 // planes (1 KiB aligned), then the raw rows and the norm weight; 0 when that
@@ -575,7 +578,7 @@ size_t fused_lds_bytes(const DevWeight& w, const XSrc& src, int m) {
     const int K = src.K ? src.K : w.cols;
     if (K != w.cols || K % 4 || src.ldx % 4 || (uintptr_t)src.x % 16) return 0;
     if (src.mode == XS_NORM && (!src.w || (uintptr_t)src.w % 16)) return 0;
-    const size_t planes = (lds_bytes(w, m) + 1023) & ~(size_t)1023;
+    const size_t planes = lds_bytes(w, m);
     size_t raw = ((size_t)(m + (src.mode == XS_NORM ? 1 : 0)) * K * 4 + 1023) & ~(size_t)1023;
     if (src.mode == XS_CAT) {
         const int H = src.H;
@@ -688,7 +691,7 @@ static int launch_args(const DevWeight& w, GemvArgs& a, int ks_override, int gri
         // scales, rounded to whole 1 KiB direct-load chunks
         if (w.dtype != DT_Q8ROW || a.src.cs_ld != w.kchunks || grouped)
             return fail("gemv: chunk-scaled operands are q8, contiguous, ungrouped");
-        lds = ((lds_bytes(w, m) + 1023) & ~(size_t)1023) + (((size_t)m * w.kchunks * 4 + 1023) & ~(size_t)1023);
+        lds = lds_bytes(w, m) + (((size_t)m * w.kchunks * 4 + 1023) & ~(size_t)1023);
         if (lds > LDSX_MAX) return fail("gemv: chunk-scaled operand too large for LDS");
         xm = XM_PREPC;
     } else if (a.src.mode == XS_GLOBAL) {
