@@ -175,8 +175,9 @@ __global__ __launch_bounds__(256) void k_prefill_fakv(const float* __restrict__ 
 // blocks see different numbers of tiles, so blocks are paired, i with z =
 // nqb - 1 - i, and a pair's tiles dealt to two workgroups evenly: unit 2 i
 // takes the first half of them (all block z's, the longer), unit 2 i + 1 the
-// rest of z's and then block i's.  The halves of z meet through pt / pml: the
-// unit that ends second (mcell's exchange finds the launch's tag) takes the
+// rest of z's and then block i's.  The halves of z meet through pt / pml: each
+// wave releases its sums at agent scope, then thread 0 exchanges the launch's
+// tag into mcell; the unit that ends second (it finds the tag there) takes the
 // first one's sums and writes the rows; none waits.
 //
 // The floor is the MFMA's (48 of 32x32x16 a wave and tile: 25 us at 2048
@@ -419,6 +420,9 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
 #pragma unroll
                 for (int i = 0; i < 8; i++) mine[i * 64] = res[i];
                 if (par == 0) ml[upper * 256] = float2v{M, L};
+                // (every wave's own sums are out before the barrier that lets
+                // thread 0 publish them: the barrier alone waits for no store)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
                 __syncthreads();
                 second = seen(false);
                 if (!second) continue;
