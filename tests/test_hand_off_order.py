@@ -21,7 +21,7 @@ def test_partial_sums_are_out_before_they_are_published(tmp_path):
                         os.path.join(ROOT, "cmf_amd", "csrc", "prefill_attn.hip"), "-o", str(out)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    kernels = re.findall(r"^(_Z\S*k_prefill_fa\S*):(.*?)s_endpgm", out.read_text(), re.S | re.M)
+    kernels = re.findall(r"^(_Z\S*k_prefill_faI\S*):(.*?)\.Lfunc_end", out.read_text(), re.S | re.M)
     assert len(kernels) == 10
     for name, body in kernels:
         code = [l.strip() for l in body.splitlines()]
