@@ -809,9 +809,11 @@ int cmf_gemv_dev_noalloc(cmf_weight w, const float* d_x, int ldx, int b, float* 
     if (!base) return fail("gemv_dev_noalloc: no workspace on this device");
     float* xs = (float*)(base + NOALLOC_PLANES_MAX);
     hipStream_t st = stream();
-    if (b == 1 && gemv_m1x_ok(w->w, d_x)) {
-        // one launch: the kernel stages its operand from the f32 row (the
-        // same planes, so the same result bit for bit)
+    // one launch: the kernel stages its operand from the f32 row (the same
+    // planes, so the same result bit for bit).  Every workgroup of it reads the
+    // whole row, so a result that overlaps the row takes the prepared operand.
+    const bool apart = d_y + w->w.rows <= d_x || d_x + w->w.cols <= d_y;
+    if (b == 1 && apart && gemv_m1x_ok(w->w, d_x)) {
         XSrc src{};
         src.mode = XS_ROWS;
         src.x = d_x;
