@@ -602,28 +602,45 @@ int ensure_prefill_bufs(cmf_model_s* m) {
     return CMF_OK;
 }
 
-// The scratch of the routed-expert blocks' prefill: for the widest of them.
-int ensure_prefill_moe(cmf_model_s* m) {
-    const int R = std::min(prefill_chunk(), m->c.max_seq);
+// Whether l's routed experts run as large-batch GEMMs over cnt prefill rows:
+// more rows than a verify batch, operands that have a producer, and scratch.
+bool prefill_moe_ok(cmf_model_s* m, const LayerDev& l, int cnt) {
+    return cnt > MAXB && moe_prefill_ok(l.moe, src_norm(m->pf_h, m->c.hidden, l.post_norm, m->c.eps)) &&
+           m->pf_moe_cap >= moe_prefill_scratch(l.moe, std::min(cnt, moe_prefill_tokens(l.moe))) &&
+           m->pf_rlog_cap >= (size_t)cnt * l.n_experts * sizeof(float);
+}
+
+// The scratch of the routed-expert blocks' prefill of n positions: for the
+// widest of them, in steps of 256 rows (128 experts of 2048/768: 168 MB at 256
+// rows, 403 MB at 2048).  Where it does not fit, the rows go 16 at a time
+// (prefill_moe_ok; CMF_PREFILL_MOE_FAIL=1 refuses it, to test that path).
+void ensure_prefill_moe(cmf_model_s* m, int n) {
+    if (std::min(n, prefill_chunk()) <= MAXB) return;
+    const int R = std::min((n + 255) / 256 * 256, std::min(prefill_chunk(), m->c.max_seq));
     size_t need = 0, rl = 0;
     for (auto& l : m->L)
-        if (l.moe) {
+        if (l.moe && moe_prefill_ok(l.moe, src_norm(m->pf_h, m->c.hidden, l.post_norm, m->c.eps))) {
             need = std::max(need, moe_prefill_scratch(l.moe, std::min(R, moe_prefill_tokens(l.moe))));
             rl = std::max(rl, (size_t)R * l.n_experts);
         }
-    auto grow = [&](void** p, size_t* cap, size_t bytes) -> int {
-        if (*cap >= bytes) return CMF_OK;
-        if (*p) {  // (a layer was replaced by a wider one)
+    static const bool refuse = getenv("CMF_PREFILL_MOE_FAIL") && getenv("CMF_PREFILL_MOE_FAIL")[0] == '1';
+    auto grow = [&](void** p, size_t* cap, size_t bytes) {
+        if (*cap >= bytes) return;
+        if (*p) {
             m->allocs.erase(std::find(m->allocs.begin(), m->allocs.end(), *p));
             (void)hipFree(*p);
             *p = nullptr;
             *cap = 0;
         }
-        if (dalloc(m, p, bytes)) return CMF_ERR;
+        if (refuse || dalloc(m, p, bytes)) {
+            *p = nullptr;
+            (void)hipGetLastError();
+            return;
+        }
         *cap = bytes;
-        return CMF_OK;
     };
-    return grow(&m->pf_moe, &m->pf_moe_cap, need) || grow((void**)&m->pf_rlog, &m->pf_rlog_cap, rl * sizeof(float)) ? CMF_ERR : CMF_OK;
+    grow(&m->pf_moe, &m->pf_moe_cap, need);
+    grow((void**)&m->pf_rlog, &m->pf_rlog_cap, rl * sizeof(float));
 }
 
 // Causal attention of cnt chunk rows (positions *pb + i) in groups the
@@ -696,7 +713,7 @@ int prefill_block(cmf_model_s* m, LayerDev& l, float* h, int cnt, const int* pb,
     ra.ldx = nh * hd;
     if ((rc = gemm(l.wo, ra, cnt, h, H, true, s)) != CMF_OK) return rc;
     if (l.moe) {
-        if (cnt > MAXB && moe_prefill_ok(l.moe, src_norm(h, H, l.post_norm, c.eps))) return prefill_moe(m, l, h, cnt, s);
+        if (prefill_moe_ok(m, l, cnt)) return prefill_moe(m, l, h, cnt, s);
         // the routed experts in batches of 16 rows (the verify-batch kernels)
         for (int b0 = 0; b0 < cnt; b0 += MAXB)
             if ((rc = moe_block_ffn(m, l, h + (size_t)b0 * H, std::min(MAXB, cnt - b0), s))) return rc;
@@ -1023,7 +1040,8 @@ static int ready(cmf_model m) {
 int cmf_prefill(cmf_model m, const int32_t* ids, int n) {
     if (ready(m)) return CMF_ERR;
     if (!ids || n < 1 || n + 1 > m->c.max_seq) return fail("prefill: 1 <= n < max_seq");
-    if (ensure_prefill_bufs(m) || ensure_prefill_moe(m)) return CMF_ERR;
+    if (ensure_prefill_bufs(m)) return CMF_ERR;
+    ensure_prefill_moe(m, n);
     for (int i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= m->c.vocab) return fail("prefill: token id out of range");
     hipStream_t s = stream();

@@ -1284,8 +1284,8 @@ int cmf::moe_ffn_launch(cmf_moe m, const XSrc& x, const float* d_logits, int b, 
     return moe_experts(m, x, b, m->top_k, d_out, ldo, resid, s, true, true);
 }
 
-// Prefill rows: at most 16384 pairs a call (config-5 experts: 24576 rows with
-// the tiles' padding, 200 MB of operand planes and 350 of outputs; more
+// Prefill rows: at most 16384 pairs a call (128 experts of 2048/768: 24576 rows with
+// the tiles' padding, 200 MB of operand planes and 200 of outputs; more
 // rows a call would no longer save weight reads).
 int cmf::moe_prefill_tokens(cmf_moe m) { return std::max(MAXB, 16384 / m->top_k); }
 static int moe_prefill_maxtiles(cmf_moe m, int T) {
