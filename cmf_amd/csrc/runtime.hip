@@ -550,16 +550,19 @@ int cmf_ffn(cmf_weight w1, cmf_weight w3, cmf_weight w2, const float* xs, int b,
     hipStream_t st = stream();
     // batches above 16 rows: the large-batch GEMMs over whole chunks (one
     // read of each weight and one pair of host copies a chunk, instead of
-    // one a 16-row batch: 2048x6144 q4tp, 200 rows 1045 -> 200 us)
-    if (b > MAXB && hidden <= 16384 && inter <= 16384) {
+    // one a 16-row batch: 2048x6144 q4tp, 200 rows 1065 -> 331 us).  Rows whose
+    // scratch does not fit (2048 rows of 4096x12288: 370 MB) go 16 at a time.
+    // (CMF_FFN_GEMM=0: all of them)
+    static const bool large_env = !(getenv("CMF_FFN_GEMM") && getenv("CMF_FFN_GEMM")[0] == '0');
+    int done = 0;
+    if (b > MAXB && hidden <= 16384 && inter <= 16384 && large_env) {
         const int R = std::min(b, 2048);
-        if (grow((void**)&g_ss.x, &g_ss.x_cap, (size_t)R * hidden * sizeof(float)) != CMF_OK ||
-            grow((void**)&g_ss.gu, &g_ss.gu_cap, (size_t)R * 2 * inter * sizeof(float)) != CMF_OK ||
-            grow((void**)&g_ss.y, &g_ss.y_cap, (size_t)R * hidden * sizeof(float)) != CMF_OK)
-            return CMF_ERR;
-        for (int b0 = 0; b0 < b; b0 += R) {
-            const int m = std::min(R, b - b0);
-            CMF_HIP(hipMemcpyAsync(g_ss.x, xs + (size_t)b0 * hidden, (size_t)m * hidden * 4, hipMemcpyHostToDevice, st));
+        bool ok = grow((void**)&g_ss.x, &g_ss.x_cap, (size_t)R * hidden * sizeof(float)) == CMF_OK &&
+                  grow((void**)&g_ss.gu, &g_ss.gu_cap, (size_t)R * 2 * inter * sizeof(float)) == CMF_OK &&
+                  grow((void**)&g_ss.y, &g_ss.y_cap, (size_t)R * hidden * sizeof(float)) == CMF_OK;
+        while (ok && done < b) {
+            const int m = std::min(R, b - done);
+            CMF_HIP(hipMemcpyAsync(g_ss.x, xs + (size_t)done * hidden, (size_t)m * hidden * 4, hipMemcpyHostToDevice, st));
             XSrc rx{};
             rx.mode = XS_ROWS;
             rx.x = g_ss.x;
@@ -569,15 +572,20 @@ int cmf_ffn(cmf_weight w1, cmf_weight w3, cmf_weight w2, const float* xs, int b,
             sg.x = g_ss.gu;
             sg.ldx = 2 * inter;
             sg.K = inter;
-            if (gemm(w1->w, rx, m, g_ss.gu, 2 * inter, false, st) != CMF_OK ||
-                gemm(w3->w, rx, m, g_ss.gu + inter, 2 * inter, false, st, true) != CMF_OK ||
-                gemm(w2->w, sg, m, g_ss.y, hidden, false, st) != CMF_OK)
-                return CMF_ERR;
-            CMF_HIP(hipMemcpyAsync(out + (size_t)b0 * hidden, g_ss.y, (size_t)m * hidden * 4, hipMemcpyDeviceToHost, st));
+            ok = gemm(w1->w, rx, m, g_ss.gu, 2 * inter, false, st) == CMF_OK &&
+                 gemm(w3->w, rx, m, g_ss.gu + inter, 2 * inter, false, st, true) == CMF_OK &&
+                 gemm(w2->w, sg, m, g_ss.y, hidden, false, st) == CMF_OK;
+            if (!ok) break;
+            CMF_HIP(hipMemcpyAsync(out + (size_t)done * hidden, g_ss.y, (size_t)m * hidden * 4, hipMemcpyDeviceToHost, st));
+            done += m;
         }
-        CMF_HIP(hipStreamSynchronize(st));
-        CMF_HIP(hipGetLastError());
-        return CMF_OK;
+        if (done >= b) {
+            CMF_HIP(hipStreamSynchronize(st));
+            CMF_HIP(hipGetLastError());
+            return CMF_OK;
+        }
+        (void)hipStreamSynchronize(st);
+        (void)hipGetLastError();
     }
     // device buffers (the thread's grow-only seam scratch): x [m][hidden],
     // g/u [m][2*inter], planes, out [m][hidden]
@@ -591,7 +599,7 @@ int cmf_ffn(cmf_weight w1, cmf_weight w3, cmf_weight w2, const float* xs, int b,
     float *dx = g_ss.x, *dgu = g_ss.gu, *dy = g_ss.y, *dxs = g_ss.xs;
     uint8_t* pl = g_ss.planes;
     int rc = CMF_OK;
-    for (int b0 = 0; b0 < b && rc == CMF_OK; b0 += MAXB) {
+    for (int b0 = done; b0 < b && rc == CMF_OK; b0 += MAXB) {
         const int m = std::min(MAXB, b - b0);
         CMF_HIP(hipMemcpyAsync(dx, xs + (size_t)b0 * hidden, (size_t)m * hidden * 4, hipMemcpyHostToDevice, st));
         launch_prep(w1->w, dx, hidden, m, pl, dxs, st);
