@@ -283,6 +283,7 @@ static int grow(void** p, size_t* cap, size_t need) {
     if (*cap >= need) return CMF_OK;
     if (*p) (void)hipFree(*p);
     *p = nullptr;
+    *cap = 0;  // (a refused allocation leaves none)
     CMF_HIP(hipMalloc(p, need));
     *cap = need;
     return CMF_OK;
