@@ -159,6 +159,7 @@ struct cmf_model_s {
     hipGraphExec_t plain_graph = nullptr;  // one captured plain step
     int plain_len = 0;
     int plain_sampling = -1;
+    unsigned long long moe_ver = 0;  // expert uploads that the captured rounds have seen
     cmf_spec_state mon{};  // the speculation monitor of the last cmf_decode (spec = 2)
     bool use_graph = true;
     bool decoding = false;
@@ -1030,10 +1031,16 @@ static int xl_restore(cmf_model m, const XlSnap& sn) {
 static int ready(cmf_model m) {
     if (!m) return fail("null model");
     if (!m->has_head) return fail("model has no lm_head (cmf_model_set_head)");
+    unsigned long long ver = 0;
     for (auto& l : m->L) {
         if (!l.qkv.w) return fail("model has unset layers (cmf_model_set_layer)");
         if (l.moe && moe_prepare(l.moe) != CMF_OK) return CMF_ERR;  // before any captured round
+        ver += moe_version(l.moe);
     }
+    // (an expert set again may have another codec: the captured kernels are
+    // those of the one before)
+    if (ver != m->moe_ver) drop_graph(m);
+    m->moe_ver = ver;
     return CMF_OK;
 }
 

@@ -1086,6 +1086,7 @@ struct cmf_moe_s {
     GemvDesc* d_gu = nullptr;  // device descriptor arrays [ne]
     GemvDesc* d_down = nullptr;
     bool desc_ok = false;
+    unsigned long long version = 0;  // expert uploads so far
     // device scratch
     float *x = nullptr, *logits = nullptr, *w = nullptr, *out = nullptr;
     int *idx = nullptr, *jobs = nullptr, *slot = nullptr, *jt = nullptr;
@@ -1261,6 +1262,7 @@ static XSrc rows_src(const float* d_x, int H) {
 int cmf::moe_prepare(cmf_moe m) { return moe_ready(m); }
 int cmf::moe_hidden(cmf_moe m) { return m ? m->hidden : 0; }
 int cmf::moe_experts_count(cmf_moe m) { return m ? m->ne : 0; }
+unsigned long long cmf::moe_version(cmf_moe m) { return m ? m->version : 0; }
 
 int cmf::moe_ffn_launch(cmf_moe m, const XSrc& x, const float* d_logits, int b, float* d_out, int ldo, bool resid,
                    hipStream_t s) {
@@ -1457,6 +1459,7 @@ int cmf_moe_set_expert(cmf_moe m, int e, const cmf_tensor* gate, const cmf_tenso
     m->down[e] = dn;
     m->set[e] = 1;
     m->desc_ok = false;
+    m->version += 1;
     return CMF_OK;
 }
 

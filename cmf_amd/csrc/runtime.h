@@ -42,6 +42,7 @@ struct XSrc;
 int moe_prepare(cmf_moe_s* m);
 int moe_hidden(cmf_moe_s* m);
 int moe_experts_count(cmf_moe_s* m);
+unsigned long long moe_version(cmf_moe_s* m);  // counts cmf_moe_set_expert calls
 int moe_ffn_launch(cmf_moe_s* m, const XSrc& x, const float* d_logits, int b, float* d_out, int ldo, bool resid,
                    hipStream_t s);
 // The same for T > 16 rows (a prefill chunk): every (token, expert) pair in

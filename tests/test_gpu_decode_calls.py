@@ -53,3 +53,27 @@ def test_bad_draft_count_is_refused(gpu, calls, k):
             m.decode(12, spec=spec, k=k)
     assert len(m.decode(12, spec=False, k=k)[0]) == 12  # (plain steps take no drafts)
     m.free()
+
+
+def test_expert_of_another_codec_after_a_decode(gpu):
+    """the one expert of a routed layer, set again in another codec between
+    two decodes: the second runs its kernels, not those captured before"""
+    import ctypes as C
+
+    from cmf_amd import DT_Q4T, DT_Q8ROW, check, lib, synth
+    from cmf_amd.model import Model, _tensor
+    moe = dict(n_experts=1, top_k=1, inter=128, layers=[0, 1], router_dtype="q8")
+    sms = [synth.synth_model(CFG, seed=31, norm_noise=0.3, sigma=0.08, mtp=False, moe=moe, ffn_dtype=dt) for dt in (DT_Q8ROW, DT_Q4T)]
+    prompt = synth.ids(34, 12, CFG["vocab"])
+    want = []
+    for sm in sms:
+        m = Model(sm)
+        want.append(_decode(m, prompt, 16, spec=False))
+        m.free()
+    m = Model(sms[0])
+    assert _decode(m, prompt, 16, spec=False) == want[0]
+    for layer, li in zip(m.moes, (0, 1)):
+        ex, keep = sms[1]["layers"][li]["moe"]["experts"][0], []
+        check(lib().cmf_moe_set_expert(layer.h, 0, *(C.byref(_tensor(ex[n], keep)) for n in ("gate", "up", "down"))))
+    assert _decode(m, prompt, 16, spec=False) == want[1]
+    m.free()
