@@ -26,7 +26,7 @@ def test_each_call_uses_its_sampler(gpu, calls, spec, n, k):
     from cmf_amd import SamplerConfig
     from cmf_amd.model import Model
     sm, prompt = calls
-    samplers = [SamplerConfig(0.8, 0.9, 1, 1.0, 0.05), SamplerConfig(1.5, 1.0, 64, 1.0, 0.0), SamplerConfig(1.5, 0.3, 64, 1.0, 0.0)]
+    samplers = [SamplerConfig(0.8, 0.9, 1, 1.0, 0.05), SamplerConfig(1.5, 1.0, 64, 1.0, 0.0), SamplerConfig(0.3, 0.1, 40, 1.0, 0.0)]
     fresh = []
     for s in samplers:
         m = Model(sm)
