@@ -21,9 +21,15 @@ def _model():
 
 
 def test_scratch_follows_the_prompt(gpu):
-    import torch
+    import ctypes as C
+
     from cmf_amd import synth
-    free = lambda: torch.cuda.mem_get_info()[0]  # noqa: E731
+    hip = C.CDLL("libamdhip64.so.7")  # (the one the library is linked to)
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
     m = _model()
     ids = synth.ids(32, 2100, CFG["vocab"])
     m.prefill(ids)  # (the thread's GEMM operands)
