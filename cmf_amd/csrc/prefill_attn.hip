@@ -175,10 +175,12 @@ __global__ __launch_bounds__(256) void k_prefill_fakv(const float* __restrict__ 
 // blocks see different numbers of tiles, so blocks are paired, i with z =
 // nqb - 1 - i, and a pair's tiles dealt to two workgroups evenly: unit 2 i
 // takes the first half of them (all block z's, the longer), unit 2 i + 1 the
-// rest of z's and then block i's.  The halves of z meet through pt / pml: each
-// wave releases its sums at agent scope, then thread 0 exchanges the launch's
-// tag into mcell; the unit that ends second (it finds the tag there) takes the
-// first one's sums and writes the rows; none waits.
+// rest of z's and then block i's.  The halves of z meet through pt / pml: every
+// wave waits until its sums are in L2, thread 0 writes that back (the other
+// unit may be on another XCD; a release by each wave instead costs 15 us at
+// 2048 positions) and exchanges the launch's tag into mcell; the unit that ends
+// second (it finds the tag there) takes the first one's sums and writes the
+// rows; none waits.
 //
 // The floor is the MFMA's (48 of 32x32x16 a wave and tile: 25 us at 2048
 // positions of 16 heads at 2 GHz).  Against 64-row blocks of four 16-row
@@ -409,8 +411,12 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
             float2v* ml = pml + 2 * cell * 256 + wave * 64 + ln;  // (both halves' waves hold them)
             const auto seen = [&](bool first) {
                 if (t == 0) {
+                    if (!first) {  // write the XCD's L2 back; the exchange goes out after that
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    }
                     s_second = (first ? __hip_atomic_load(mcell + cell, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)
-                                      : __hip_atomic_exchange(mcell + cell, tag, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT)) == tag;
+                                      : __hip_atomic_exchange(mcell + cell, tag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)) == tag;
                 }
                 __syncthreads();
                 return s_second != 0;
@@ -420,9 +426,10 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
 #pragma unroll
                 for (int i = 0; i < 8; i++) mine[i * 64] = res[i];
                 if (par == 0) ml[upper * 256] = float2v{M, L};
-                // (every wave's own sums are out before the barrier that lets
-                // thread 0 publish them: the barrier alone waits for no store)
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                // (every wave's own sums are in L2 before the barrier that lets
+                // thread 0 release and publish them: the barrier alone waits
+                // for no store)
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
                 second = seen(false);
                 if (!second) continue;

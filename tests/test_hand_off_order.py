@@ -2,7 +2,8 @@
 global memory: the one that publishes its sums (an exchange of the launch's
 tag by one thread, after a workgroup barrier) must have had every wave's
 stores finished before that barrier.  On gfx950 the barrier itself waits for
-LDS only, so the wait has to stand in the code of all waves before it."""
+LDS only, so the wait has to stand in the code of all waves before it, and the
+write-back of the L2 has to have ended before the exchange."""
 import os
 import re
 import subprocess
@@ -35,5 +36,7 @@ def test_partial_sums_are_out_before_they_are_published(tmp_path):
             store = max(j for j in range(bar) if code[j].startswith("global_store"))
             wait = [c for c in code[store + 1:bar] if c.startswith("s_waitcnt") and "vmcnt(0)" in c]
             assert wait, f"{name}: no wait for the stores before the barrier"
+            back = max(j for j in range(i) if code[j].startswith("buffer_wbl2"))
+            assert back > bar and any(c.startswith("s_waitcnt") and "vmcnt(0)" in c for c in code[back + 1:i]), name
             published += 1
         assert published == 1, name
