@@ -8,9 +8,10 @@
 //     kernels do it;
 //   - k_prefill_fakv: the cache's K / V rows [0, p0 + cnt) rearranged into
 //     32-key tiles of the attention's MFMA fragments (f16 hi / lo halves);
-//   - k_prefill_fa: 128 query rows per block, two blocks per two workgroups,
-//     each tile in LDS once per workgroup, with a running (online)
-//     softmax: scores on the f16 MFMA (q.k = qh.kh + qh.kl + ql.kh, 22-bit
+//   - k_prefill_fa: 128 query rows per block, two blocks per two workgroups
+//     (contexts of at most FA64_KEYS: k_prefill_fa64, 64 rows per block, two
+//     blocks per workgroup), each tile in LDS once per workgroup, with a
+//     running (online) softmax: scores on the f16 MFMA (q.k = qh.kh + qh.kl + ql.kh, 22-bit
 //     operands, f32 sums), causal limit the row's position
 //     (kv_cache.rs:521-690), values ph.vh + ph.vl + pl.vh on the f16 MFMA.
 // Rows of a block past the chunk see no keys and write nothing.
@@ -36,6 +37,8 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 constexpr int HD = 128;
 constexpr int KT2 = 128;      // the K / V scratch's padding unit (keys)
 
+__device__ __forceinline__ void wait_vmcnt0() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }  // vmcnt(0) only
+__device__ __forceinline__ void wait_vmcnt4() { __builtin_amdgcn_s_waitcnt(4 | (7 << 4) | (15 << 8)); }  // vmcnt(4) only
 __device__ __forceinline__ void wait_all() { __builtin_amdgcn_s_waitcnt(7 << 4); }  // vmcnt(0) lgkmcnt(0)
 
 // the LDS reads before the last N are in
@@ -49,6 +52,22 @@ __device__ __forceinline__ uint32_t xcc_id() {
     uint32_t v;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID, 0, 4)" : "=s"(v));
     return v;
+}
+
+// max / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (one MFMA output
+// column) by the gfx950 row-swap permutes: each returns the value and its
+// partner's, so op(first, second) is the pairwise result in every lane
+__device__ __forceinline__ float lanes4_max(float v) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float lanes4_sum(float v) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
 // max / sum over the lanes l, l ^ 32 (one column of a 32x32 MFMA output) by
@@ -113,16 +132,28 @@ constexpr int FT = 32;                // keys per tile
 constexpr int FT_BYTES = 32 * 1024;   // one tile of one kv head: K then V fragments
 constexpr int FQ = 128;               // query rows per block
 constexpr int FRA = 4;                // fragment pairs read ahead
+// contexts of at most this many keys take the 64-row blocks of 16-row waves
+// (k_prefill_fa64): us a layer, 64 rows / 128 rows, of 16 query heads on 8 KV
+// heads: 64 keys 8.7 / 13.8, 128 12 / 21, 256 16 / 23, 512 25.6 / 27.4, 640
+// 30.7 / 29.7, 1024 45 / 36, 2048 86 / 59 (8 on 8, 4 on 4: 512 25.6 / 27,
+// 640 30 / 29 and 31.9 / 29)
+constexpr int FA64_KEYS = 576;
 
 // The cached K / V rows [0, n) of every kv head as 32-key tiles of MFMA
 // fragments, [nkv][npad / 32][32 fragments][64 lanes] x 16 B (keys past n
-// zero):
+// zero).  W32 (k_prefill_fa):
 //   K fragment 2 ks + plane: lane 32 h + r holds dims 16 ks + 8 h .. + 7 of
 //     key r (A operand of S^T, f16 hi / lo);
 //   V fragment 16 + 4 db + 2 t + plane: lane 32 h + r holds dim 32 db + r of
 //     the keys 16 t + 4 h + j (j < 4) and 16 t + 8 + 4 h + j - 4 (j >= 4) (A
 //     operand of O^T = V^T P^T).
+// else (k_prefill_fa64):
+//   K fragment 8 kb + 2 ks + plane: lane 16 s + r holds dims 32 ks + 8 s .. + 7
+//     of key 16 kb + r;
+//   V fragment 16 + 2 db + plane: lane 16 s + r holds dim 16 db + r of the
+//     keys 4 s + j (j < 4) and 16 + 4 s + j - 4 (j >= 4).
 // grid (npad / 32, nkv), 256 threads.
+template <bool W32>
 __global__ __launch_bounds__(256) void k_prefill_fakv(const float* __restrict__ kc, const float* __restrict__ vc,
                                                       int max_seq, int n, int npad, int4v* __restrict__ op) {
     const int t = threadIdx.x, tile = blockIdx.x, g = blockIdx.y;
@@ -141,23 +172,23 @@ __global__ __launch_bounds__(256) void k_prefill_fakv(const float* __restrict__ 
     __syncthreads();
     int4v* dst = op + ((size_t)g * (npad / FT) + tile) * (FT_BYTES / 16);
     for (int e = t; e < 32 * 64; e += 256) {
-        const int l = e & 63, f = e >> 6, r = l & 31, sl = l >> 5, plane = f & 1;
+        const int l = e & 63, f = e >> 6, r = W32 ? l & 31 : l & 15, sl = W32 ? l >> 5 : l >> 4, plane = f & 1;
         half8 h;
         if (f < 16) {
-            const int ks = f >> 1;
+            const int k = W32 ? r : 16 * (f >> 3) + r, d0 = W32 ? 16 * (f >> 1) + 8 * sl : 32 * ((f >> 1) & 3) + 8 * sl;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 _Float16 hh, ll;
-                split16(KS[r][16 * ks + 8 * sl + j], hh, ll);
+                split16(KS[k][d0 + j], hh, ll);
                 h[j] = plane ? ll : hh;
             }
         } else {
-            const int db = (f - 16) >> 2, kt = (f >> 1) & 1;
+            const int d = W32 ? 32 * ((f - 16) >> 2) + r : 16 * ((f - 16) >> 1) + r;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const int k = 16 * kt + 8 * (j >> 2) + 4 * sl + (j & 3);
+                const int k = W32 ? 16 * ((f >> 1) & 1) + 8 * (j >> 2) + 4 * sl + (j & 3) : 16 * (j >> 2) + 4 * sl + (j & 3);
                 _Float16 hh, ll;
-                split16(VS[k][32 * db + r], hh, ll);
+                split16(VS[k][d], hh, ll);
                 h[j] = plane ? ll : hh;
             }
         }
@@ -183,15 +214,15 @@ __global__ __launch_bounds__(256) void k_prefill_fakv(const float* __restrict__ 
 // rows; none waits.
 //
 // The floor is the MFMA's (48 of 32x32x16 a wave and tile: 25 us at 2048
-// positions of 16 heads at 2 GHz).  Against 64-row blocks of four 16-row
-// waves, a pair a workgroup (87 -> 63 us): 32 rows a wave halve the LDS reads
-// per MFMA, both waves of a SIMD have work to the end (the pair's short
-// block left four of the eight waves idle past its keys), and the tiles cross
-// L2 8448 times instead of 12416.  What is left beside the MFMA is spread:
-// without the tile fetch, the LDS reads or the softmax (timing only) it takes
-// 57 to 61 us each; about 13 us are the rows' loads, the two merges and the
-// stores.  Not better: the last tile's values in the shadow of the next
-// softmax (65 us), rows staged through LDS (63).
+// positions of 16 heads at 2 GHz).  Against k_prefill_fa64 (86 -> 59 us): 32
+// rows a wave halve the LDS reads per MFMA, both waves of a SIMD have work to
+// the end (the pair's short block left four of the eight waves idle past its
+// keys), and the tiles cross L2 8448 times instead of 12416.  What is left
+// beside the MFMA is spread: without the tile fetch, the LDS reads or the
+// softmax (timing only, of a build that took 63 us) it takes 57 to 61 us each;
+// about 13 us are the rows' loads, the two merges and the stores.  Not better
+// than that build: the last tile's values in the shadow of the next softmax
+// (65 us), rows staged through LDS (63).
 //
 // XCD: the kv head is the XCD the workgroup runs on (its K / V stays in that
 // XCD's L2), which covers each (unit, head) once only while the dispatcher
@@ -457,6 +488,162 @@ __global__ __launch_bounds__(512) void k_prefill_fa(const float* __restrict__ qb
     }
 }
 
+// ---------------------------------------------------------------------------
+// Short contexts: blocks of 64 query rows in four waves of 16 (16x16x32 MFMA),
+// S^T and O^T as above with lane (query r = lane & 15, k-slot s = lane >> 4)
+// holding the weights of the keys 4 s .. + 3 and 16 + 4 s .. + 3.  Half the
+// rows and keys of a step and nothing to merge: where there are few tiles the
+// fixed costs of k_prefill_fa (two merges, wider rows) outweigh its rate.  Bound
+// by latency: a chain of one fetch, two products and a softmax a tile.
+// grid (8 np) (XCD: kv head = the workgroup's XCD, pair index i =
+// blockIdx / 8) or (np, nkv), np = ceil(nqb / 2); 512 threads.  The
+// workgroup serves two 64-row query blocks that see about as many keys
+// together as any other pair: waves 0-3 block i, waves 4-7 block nqb - 1 -
+// i (none when that is block i again), sharing one fetch of every K / V
+// tile the short block needs.  Wave w of a block holds 16 query rows, PPW =
+// 16 / HPK positions times the HPK query heads of kv head g (row q: chunk
+// row PPW (4 qb + w % 4) + q % PPW, query head g HPK + q / PPW).  XCD: the
+// kv head is the XCD the workgroup runs on (its K / V stays in that XCD's
+// L2), which covers each (query block, head) once only while the
+// dispatcher deals workgroups to the 8 XCDs in turn; each workgroup
+// therefore swaps the launch's tag into its blocks' cells [qb][g] first,
+// and finding the tag already there sets *perr: the host then re-runs the
+// prefill on the grid-indexed variant.
+template <int HPK, bool XCD>
+__global__ __launch_bounds__(512) void k_prefill_fa64(const float* __restrict__ qbuf, const int4v* __restrict__ op,
+                                                    int npad, int cnt, int p0, int nh, int nqb, float* __restrict__ out,
+                                                    unsigned long long* cells, int* perr, unsigned long long tag) {
+    constexpr int PPW = 16 / HPK;
+    extern __shared__ __align__(16) uint8_t fsm[];  // three tiles (direct-load targets)
+    const int pi = XCD ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    const int g = XCD ? (int)(xcc_id() & 7) : (int)blockIdx.y;
+    const int qa = pi, qz = nqb - 1 - pi;  // the pair (qz == qa: one block)
+    if constexpr (XCD) {
+        if (threadIdx.x == 0 && atomicExch(cells + qa * 8 + g, tag) == tag) atomicOr(perr, 1);
+        if (threadIdx.x == 64 && qz != qa && atomicExch(cells + qz * 8 + g, tag) == tag) atomicOr(perr, 1);
+    }
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int r = lane & 15, s = lane >> 4;
+    const bool second = wave >= 4;
+    const bool live = !second || qz != qa;                 // (uniform per wave)
+    const int qb = second ? qz : qa;
+    const int i0 = (4 * qb + (wave & 3)) * PPW;           // this wave's first chunk row
+    const int lastrow = min((4 * qb + 4) * PPW, cnt) - 1; // its block's last chunk row
+    const int lastz = min((4 * max(qa, qz) + 4) * PPW, cnt) - 1;  // the pair's
+    // the queries of column r (the B operand of S^T), f16 hi / lo
+    const bool qv = live && i0 + r % PPW < cnt;
+    const int qpos = p0 + i0 + r % PPW;                 // position of query r
+    half8 qh[HD / 32], ql[HD / 32];
+    {
+        const float* qrow = qbuf + ((size_t)(qv ? i0 + r % PPW : 0) * nh + g * HPK + r / PPW) * HD;
+#pragma unroll
+        for (int ks = 0; ks < HD / 32; ks++) {
+            const float4v a0 = *(const float4v*)(qrow + 32 * ks + 8 * s);
+            const float4v a1 = *(const float4v*)(qrow + 32 * ks + 8 * s + 4);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                _Float16 hh, ll;
+                split16(qv ? (j < 4 ? a0[j] : a1[j - 4]) : 0.f, hh, ll);
+                qh[ks][j] = hh;
+                ql[ks][j] = ll;
+            }
+        }
+    }
+    // tiles of the pair (the fetch loop) and of this wave's block
+    const int ntiles = lastz < 0 ? 0 : (p0 + lastz) / FT + 1;
+    const int mytiles = !live || lastrow < 0 ? 0 : (p0 + lastrow) / FT + 1;
+    const uint8_t* src = (const uint8_t*)(op + (size_t)g * (npad / FT) * (FT_BYTES / 16));
+    // tile tt into buffer b: 32 KiB as 32 chunks of 1 KiB, 4 per wave
+    auto fetch = [&](int tt, int b) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int ch = 4 * wave + c;
+            __builtin_amdgcn_global_load_lds((const void*)(src + (size_t)tt * FT_BYTES + ch * 1024 + lane * 16),
+                                             (__attribute__((address_space(3))) void*)(fsm + b * FT_BYTES + ch * 1024),
+                                             16, 0, 0);
+        }
+    };
+    const float scale = 1.4426950408889634f / sqrtf((float)HD);
+    float m = -INFINITY, l = 0.f;   // of query r (the same in the four lanes of column r)
+    float4v o[8];                   // rows 4 s + e, dims 16 db + r
+#pragma unroll
+    for (int db = 0; db < 8; db++) o[db] = float4v{0.f, 0.f, 0.f, 0.f};
+    // three buffers: tile tt + 2 is requested while tile tt is used
+    if (ntiles > 0) fetch(0, 0);
+    if (ntiles > 1) fetch(1, 1);
+    for (int tt = 0; tt < ntiles; tt++) {
+        const int b = tt % 3;
+        if (tt + 1 < ntiles) wait_vmcnt4();  // tile tt's share is in (tile tt + 1's may not be)
+        else wait_vmcnt0();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave's share is in; tile tt - 1's buffer is free
+        if (tt + 2 < ntiles) fetch(tt + 2, (tt + 2) % 3);
+        if (tt >= mytiles) continue;  // (uniform per wave: past this block's keys)
+        const int4v* F = (const int4v*)(fsm + b * FT_BYTES) + lane;
+        // S^T for the two key blocks: d[kb][e] = key 16 kb + 4 s + e, query r
+        float4v d[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+            float4v d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0, d2 = d0;
+#pragma unroll
+            for (int ks = 0; ks < HD / 32; ks++) {
+                const half8 kh = __builtin_bit_cast(half8, F[(8 * kb + 2 * ks) * 64]);
+                const half8 kl = __builtin_bit_cast(half8, F[(8 * kb + 2 * ks + 1) * 64]);
+                d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[ks], d0, 0, 0, 0);
+                d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[ks], d1, 0, 0, 0);
+                d2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[ks], d2, 0, 0, 0);
+            }
+            d[kb] = d0 + (d1 + d2);
+        }
+        // causal mask, log2 scale, the running softmax of query r
+        float sv[8];
+        float mt = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int key = FT * tt + (j < 4 ? 4 * s + j : 16 + 4 * s + (j - 4));
+            const float x = j < 4 ? d[0][j] : d[1][j - 4];
+            sv[j] = qv && key <= qpos ? x * scale : -INFINITY;
+            mt = fmaxf(mt, sv[j]);
+        }
+        mt = lanes4_max(mt);
+        const float mn = fmaxf(m, mt);
+        const float al = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+        float ps = 0.f;
+        half8 ph, pl;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float pv = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sv[j] - mn);
+            ps += pv;
+            _Float16 hh, ll;
+            split16(pv, hh, ll);
+            ph[j] = hh;
+            pl[j] = ll;
+        }
+        ps = lanes4_sum(ps);
+        l = l * al + ps;
+        m = mn;
+        // O^T += V^T P^T (the same registers as operands the other way
+        // round): lane (query r, s) holds dims 16 db + 4 s + e of its own
+        // query, so the rescale needs no exchange
+#pragma unroll
+        for (int db = 0; db < 8; db++) {
+            float4v acc = o[db] * al;
+            const half8 vh = __builtin_bit_cast(half8, F[(16 + 2 * db) * 64]);
+            const half8 vl = __builtin_bit_cast(half8, F[(16 + 2 * db + 1) * 64]);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl, acc, 0, 0, 0);
+            o[db] = acc;
+        }
+    }
+    // out = o / l of query r: dims 16 db + 4 s .. + 3
+    const int row = i0 + r % PPW, head = g * HPK + r / PPW;
+    if (live && row < cnt) {
+        float* dst = out + (size_t)row * nh * HD + (size_t)head * HD + 4 * s;
+#pragma unroll
+        for (int db = 0; db < 8; db++) *(float4v*)(dst + 16 * db) = o[db] / l;
+    }
+}
+
 }  // namespace
 
 bool prefill_attention_fits(int nh, int nkv, int hd) {
@@ -481,12 +668,43 @@ int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(k_prefill_qk, dim3(a.cnt, hq + a.nkv), dim3(64), 0, st, a.qkv, a.ldq, a.qn, a.kn, a.rope,
                        a.kc, a.vc, a.max_seq, a.p0, a.nh, a.nkv, a.eps, a.qbuf, hq);
     if (!a.out) return CMF_OK;
-    const int hpk = a.nh / a.nkv, ppb = FQ / hpk;
+    const int hpk = a.nh / a.nkv;
     const int n = a.p0 + a.cnt, npad = (n + KT2 - 1) / KT2 * KT2;
-    const int nqb = (a.cnt + ppb - 1) / ppb;  // 128-row query blocks, paired
+    const bool small = n <= FA64_KEYS;
+    const int ppb = (small ? 64 : FQ) / hpk;
+    const int nqb = (a.cnt + ppb - 1) / ppb;  // query blocks, paired
     const int np = (nqb + 1) / 2;
     const bool xcd = a.nkv == 8 && xl_device_fits() && a.allow_xcd && a.cells && a.perr &&
-                     16 * np <= PREFILL_XCD_CELLS;
+                     (small ? 8 * nqb : 16 * np) <= PREFILL_XCD_CELLS;
+    int4v* op = (int4v*)a.khl;  // nkv x npad x 1 KiB
+    hipLaunchKernelGGL(small ? k_prefill_fakv<false> : k_prefill_fakv<true>, dim3(npad / FT, a.nkv), dim3(256), 0, st,
+                       a.kc, a.vc, a.max_seq, n, npad, op);
+    if (small) {
+        typedef void (*KernS)(const float*, const int4v*, int, int, int, int, int, float*, unsigned long long*, int*,
+                              unsigned long long);
+        KernS k;
+        switch (hpk) {
+            case 1: k = xcd ? k_prefill_fa64<1, true> : k_prefill_fa64<1, false>; break;
+            case 2: k = xcd ? k_prefill_fa64<2, true> : k_prefill_fa64<2, false>; break;
+            case 4: k = xcd ? k_prefill_fa64<4, true> : k_prefill_fa64<4, false>; break;
+            case 8: k = xcd ? k_prefill_fa64<8, true> : k_prefill_fa64<8, false>; break;
+            default: k = xcd ? k_prefill_fa64<16, true> : k_prefill_fa64<16, false>; break;
+        }
+        static const bool attr = [] {  // (96 KiB: above the default dynamic LDS limit)
+            bool ok = true;
+            for (KernS f : {k_prefill_fa64<1, true>, k_prefill_fa64<1, false>, k_prefill_fa64<2, true>,
+                            k_prefill_fa64<2, false>, k_prefill_fa64<4, true>, k_prefill_fa64<4, false>,
+                            k_prefill_fa64<8, true>, k_prefill_fa64<8, false>, k_prefill_fa64<16, true>,
+                            k_prefill_fa64<16, false>})
+                ok &= hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, 3 * FT_BYTES) ==
+                      hipSuccess;
+            return ok;
+        }();
+        if (!attr) return fail("prefill attention: dynamic LDS attribute");
+        hipLaunchKernelGGL(k, xcd ? dim3(8 * np) : dim3(np, a.nkv), dim3(512), 3 * FT_BYTES, st, a.qbuf, op, npad, a.cnt,
+                           a.p0, a.nh, nqb, a.out, a.cells, a.perr, a.tag);
+        return CMF_OK;
+    }
     typedef void (*KernF)(const float*, const int4v*, int, int, int, int, int, float*, unsigned long long*, int*,
                           unsigned long long*, unsigned long long, float4v*, float2v*);
     KernF k;
@@ -497,8 +715,6 @@ int launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st) {
         case 8: k = xcd ? k_prefill_fa<8, true> : k_prefill_fa<8, false>; break;
         default: k = xcd ? k_prefill_fa<16, true> : k_prefill_fa<16, false>; break;
     }
-    int4v* op = (int4v*)a.khl;  // nkv x npad x 1 KiB
-    hipLaunchKernelGGL(k_prefill_fakv, dim3(npad / FT, a.nkv), dim3(256), 0, st, a.kc, a.vc, a.max_seq, n, npad, op);
     const dim3 grid = xcd ? dim3(16 * np) : dim3(2 * np, a.nkv);
     static const bool attr = [] {  // (128 KiB: above the default dynamic LDS limit)
         bool ok = true;
