@@ -77,3 +77,23 @@ def test_expert_of_another_codec_after_a_decode(gpu):
         check(lib().cmf_moe_set_expert(layer.h, 0, *(C.byref(_tensor(ex[n], keep)) for n in ("gate", "up", "down"))))
     assert _decode(m, prompt, 16, spec=False) == want[1]
     m.free()
+
+
+@pytest.mark.parametrize("spec,first", [(False, 470), (True, 470), (True, 506)])
+def test_decodes_across_position_steps(gpu, spec, first, monkeypatch):
+    """decodes that cross a 512-position step, one after another at shrinking
+    and growing contexts, replay captured rounds of their own size: the tokens
+    of a model that launches every round eagerly"""
+    from cmf_amd import synth
+    from cmf_amd.model import Model
+    cfg = dict(CFG, max_seq=2400)
+    sm = synth.synth_model(cfg, seed=5, norm_noise=0.1, sigma=0.05)
+    monkeypatch.setenv("CMF_DECODE_GRAPH", "0")
+    eager = Model(sm)
+    monkeypatch.delenv("CMF_DECODE_GRAPH")
+    m = Model(sm)
+    ids = synth.ids(35, 1700, cfg["vocab"])
+    for ctx, n in ((first, 60), (1700, 20), (30, 24), (500, 40)):
+        assert _decode(m, ids[:ctx], n, spec=spec, k=4) == _decode(eager, ids[:ctx], n, spec=spec, k=4)
+    m.free()
+    eager.free()
