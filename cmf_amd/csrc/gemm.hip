@@ -610,13 +610,23 @@ int gemm(const DevWeight& w, const XSrc& src, int m, float* y, int ldy, bool res
         else hipLaunchKernelGGL((k_gemm_q8<1>), grid, dim3(256), GEMM_Q8_AT_BYTES, st, a);
         return reduce(nz);
     }
-    // 64 rows a wave (half the operand reads of 32) while that gives a
-    // workgroup to at least half the CUs, else 32: q4t 12288x4096 m = 2048
-    // 412 us at 64, 457 at 32; q4tp 6144x2048 m = 200 (96 workgroups) 50 and
-    // 40, 1000x1056 m = 77 25 and 19
-    const int rn = (long)((a.nrb + 15) / 16) * (mp / GB) >= 128 ? 2 : 1;
+    // 64 rows a wave (half the operand reads of 32) where that gives a
+    // workgroup to every CU, or to half of them and K is long enough (3072
+    // columns) for its parts to fill the rest; else 32.  Measured on MI355X, us
+    // at 64 / 32 rows: q4t 12288x4096 m = 2048 379 / 457, 4096x4096 m = 512 (128
+    // workgroups) 57 / 63, 4096x12288 m = 700 (176) 185 / 208; but 2048x2048
+    // m = 1024 (128) 40 / 35, 6144x2048 m = 512 (192) 52 / 43, 4096x1024 m = 512
+    // (128) 30 / 21; q4tp 6144x2048 m = 200 (96) 50 / 40.
+    const long wide = (long)((a.nrb + 15) / 16) * (mp / GB);
+    const int rn = wide >= 256 || (wide >= 128 && a.ntg >= 24) ? 2 : 1;
     const int rbwg = 8 * rn;
-    const int gx = (a.nrb + rbwg - 1) / rbwg, nz = split((long)gx * (mp / GB), a.ntg);
+    const int gx = (a.nrb + rbwg - 1) / rbwg;
+    // up to 11 groups of K are split only where that leaves 64 workgroups or
+    // fewer: the partial sums' launch takes 4 us (8 groups, in one part / two:
+    // q4t 3072x1024 m = 128 (48 workgroups) 19.3 / 18.7 us, 4096x1024 m = 320
+    // (160) 20 / 26, 6144x1024 m = 256 (192) 20 / 28)
+    const long base = (long)gx * (mp / GB);
+    const int nz = split(a.ntg < 12 && base > 64 ? 256 : base, a.ntg);
     if (nz < 0) return fail("gemm: split-K buffer");
     const dim3 grid(gx, mp / GB, nz);
     const bool q4t = w.dtype == DT_Q4T;
