@@ -1070,6 +1070,20 @@ MoeKernel moe_rows_pick(int dtype, int nk, bool gu, int* nw, int* rbw) {
            : dtype == DT_Q4T ? moe_rows_by_nk<DT_Q4T>(nk, gu, nw, rbw)
                              : moe_rows_by_nk<DT_Q4TP>(nk, gu, nw, rbw);
 }
+// Whether k_moe_rows beats the grouped GEMVs over all b rows: yes, except for
+// q4 rows of 2048 columns and more where the batch's jobs are many and hold a
+// token or two (us, grouped / k_moe_rows, random routing: q4tp 128 experts of
+// 2048/768, top 8, 2 tokens 33 / 33, 3 40 / 44, 4 46 / 48, 5 56 / 58, 8
+// 101 / 73; 64 of 2304/512, 4 tokens 40 / 44), and of more than 3072 where an
+// expert gets two tokens or more (8 of 4096/2048, top 2, 6 tokens 37 / 36, 7
+// 37 / 39, 8 44 / 47, 16 62 / 68).  Where all of 9 to 16 tokens pick the same
+// experts the second pass costs more than the grouped GEMVs' extra rows (32 of
+// 2048/1024, top 4, 16 tokens 29 / 45, random 84 / 58).
+bool moe_rows_pays(int dtype, int nk, int ne, int k, int b) {
+    if (dtype == DT_Q8ROW) return true;
+    if (nk >= 16 && b <= 5 && b * k >= 24) return false;
+    return !(nk > 24 && 4 * b * k >= 7 * ne);
+}
 // its dynamic LDS: the operand rows of a pass of ps slots and (q4) the tile biases
 size_t moe_rows_lds(int dtype, int nk, int ps) {
     return dtype == DT_Q8ROW ? moe_opnd_lds(ps, nk * 12) : moe_opnd_lds(ps, nk * 32) + (size_t)nk * 4 * 16 * 4;
@@ -1194,15 +1208,18 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
         d.rows = dw.rows;
         d.nrb = dw.rows_pad / 16;
         hipLaunchKernelGGL(kd, dim3((d.nrb + rw2 - 1) / rw2, mj), dim3(64 * sp2), ld, s, d);
-    } else if (MoeKernel xg = gather_env ? moe_rows_pick(gw.dtype, gw.kchunks, true, &sp1, &rw1) : nullptr,
-               xd = gather_env ? moe_rows_pick(dw.dtype, dw.kchunks, false, &sp2, &rw2) : nullptr;
+    } else if (MoeKernel xg = gather_env && moe_rows_pays(gw.dtype, gw.kchunks, m->ne, k, b)
+                                  ? moe_rows_pick(gw.dtype, gw.kchunks, true, &sp1, &rw1) : nullptr,
+               xd = xg ? moe_rows_pick(dw.dtype, dw.kchunks, false, &sp2, &rw2) : nullptr;
                xg && xd && moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks, 8)) &&
                moe_lds_ok(xd, moe_rows_lds(dw.dtype, dw.kchunks, 8))) {
         // the same two launches over each job's own tokens for any codec and
-        // up to 16 tokens; a pass holds twice the tokens that an expert gets
-        // on average (fewer slots of LDS leave room for more workgroups; a
-        // busier job takes another pass)
-        const int ps = std::min(std::min(8, b), std::max(2, (2 * b * k + m->ne - 1) / m->ne));
+        // up to 16 tokens, as many slots a pass as it holds (LDS for twice the
+        // tokens an expert gets on average was no faster on random routing:
+        // q4tp 64 experts of 1024/512, top 8, 4 tokens 29 / 24 us, 128 of
+        // 2048/768, 16 tokens 115 / 110; and 83 / 48 us there where all tokens
+        // pick the same experts, a pass for every two of them)
+        const int ps = std::min(8, b);
         MoeGx g{};
         g.desc = m->d_gu;
         g.jobs = m->jobs;
