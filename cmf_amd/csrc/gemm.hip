@@ -12,18 +12,21 @@
 //     into registers a group ahead, each wave its own rows;
 //   - the nibbles become the f16 integers n - 8 (dq_signed), so a tile needs
 //     no bias; a block of 32 x 32 outputs takes four MFMAs per tile, the lo
-//     plane's two and then the hi plane's two in one accumulator started at
-//     zero: the lo sum is exact, the hi products are integers, and the one
-//     rounding of their sum is that of the f32 add it replaces (measured on
-//     K = 4096: 2.06e-7 from an f64 product with one accumulator, 2.05e-7
-//     with two and an add); the tile scale multiplies the sum in f32 as
-//     q4t_row_exact does (qtensor.rs:4418-4432).
+//     plane's two and then the hi plane's two in one f32 accumulator started
+//     at zero; the tile scale multiplies the sum in f32 as q4t_row_exact does
+//     (qtensor.rs:4418-4432).  The lo sum is exact; each of the two hi MFMAs
+//     rounds the whole to 24 bits, where an exact accumulator per plane and an
+//     add rounded once.  That is the price of the shared accumulator: relative
+//     L2 from an f64 product 2.952e-7 -> 2.958e-7 at 512x512 m = 17, 3.123e-7
+//     -> 3.127e-7 at 2048x1024 m = 200, 0.05 to 0.2 % more wherever K has as
+//     many parts as before (3.78e-7 -> 3.73e-7 at 1024x4096 m = 200, which
+//     has more).
 // Bound by issue: per tile and block 4 MFMAs (128 cycles of the matrix
 // pipe) stand beside 16 FMAs (the tile scale) and 9 VALU ops that unpack
 // weights (100 cycles), and the clock falls to ~1.85 GHz under this load.
-// Measured on MI355X, operand preparation included: q4t 12288x4096 m = 2048
-// 571 -> 402 us, 6144x1024 123 -> 81, 1024x3072 91 -> 65, 12288x4096 m = 256
-// 123 -> 87, m = 64 57 -> 42; q4tp 12288x4096 m = 2048 891 -> 410 (the
+// Measured on MI355X (the GEMM and the sum of its parts): q4t 12288x4096 m =
+// 2048 604 -> 381 us, 6144x1024 106 -> 70, 1024x3072 64 -> 49, 12288x4096 m =
+// 256 110 -> 77, m = 64 48 -> 34; q4tp 12288x4096 m = 2048 947 -> 395 (the
 // 16x16x32 form with an accumulator per plane and tile biases from LDS took
 // 8 FMAs and adds per two MFMAs, and as many LDS as matrix cycles).
 #include <mutex>

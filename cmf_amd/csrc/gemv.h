@@ -127,7 +127,7 @@ size_t prep_bytes(const DevWeight& w);
 // xs[16] of the operand producer src for m batch rows of w.
 int launch_prep_src(const DevWeight& w, const XSrc& src, int m, uint8_t* planes, float* xs, hipStream_t st);
 // Prepared GEMM operand of m rows of the producer src: planes with row
-// stride mstride (a multiple of 64; q4: and tile biases [tile][mstride]).
+// stride mstride (a multiple of 64), without tile biases.
 int launch_prep_src_gemm(const DevWeight& w, const XSrc& src, int m, int mstride, uint8_t* planes, float* xs,
                          hipStream_t st);
 int launch_prep_rows_gemm(const DevWeight& w, const float* x, int ldx, int m, int mstride, uint8_t* planes,

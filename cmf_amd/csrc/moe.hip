@@ -24,8 +24,9 @@
 //   other codecs or larger batches (k_moe_rows, also over each job's own
 //   tokens, in passes of 5 or 8): 3. gate|up with the SwiGLU, 4. down with
 //   the operand made from the h rows in the workgroup;
-//   rows of more than 32 steps (grouped GEMVs over all b rows; rows of
-//   tokens that did not pick the expert are computed and ignored):
+//   rows of more than 32 steps, and where moe_rows_pays says so (grouped
+//   GEMVs over all b rows; rows of tokens that did not pick the expert are
+//   computed and ignored):
 //   3. gate|up, 3b. the per-job operand h = silu(g) * u, 4. down;
 //   5. k_moe_combine  out[t] = sum over ranks i of w[t][i] * down[job(t, i)][t],
 //                     accumulated from 0 in rank order, as the reference does.
@@ -1211,7 +1212,10 @@ static int moe_experts(cmf_moe m, const XSrc& x, int b, int k, float* d_out, int
     } else if (MoeKernel xg = gather_env && moe_rows_pays(gw.dtype, gw.kchunks, m->ne, k, b)
                                   ? moe_rows_pick(gw.dtype, gw.kchunks, true, &sp1, &rw1) : nullptr,
                xd = xg ? moe_rows_pick(dw.dtype, dw.kchunks, false, &sp2, &rw2) : nullptr;
-               xg && xd && moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks, 8)) &&
+               xg && xd &&
+               // (room for a full pass, whatever this batch's: q4tp rows of 4096
+               // columns keep the grouped GEMVs, 2 to 9 % slower at 1-7 tokens)
+               moe_lds_ok(xg, moe_rows_lds(gw.dtype, gw.kchunks, 8)) &&
                moe_lds_ok(xd, moe_rows_lds(dw.dtype, dw.kchunks, 8))) {
         // the same two launches over each job's own tokens for any codec and
         // up to 16 tokens, as many slots a pass as it holds (LDS for twice the

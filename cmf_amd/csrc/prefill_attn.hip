@@ -124,8 +124,9 @@ __global__ __launch_bounds__(64) void k_prefill_qk(const float* __restrict__ qkv
 // h = lane >> 5) ends up holding the weights of its own query for the keys
 // 8 b + 4 h + c: exactly the B operand of O^T = V^T P^T when the V tile's
 // k-slots hold the same keys, so the weights never go through LDS, and the
-// output's lanes hold their own query's dims.  q.k = qh.kh + qh.kl + ql.kh
-// (f16 hi / lo halves, f32 sums), exp2 of log2-scaled scores with a running
+// output's lanes hold their own query's dims.  q.k = qh.kh + (qh.kl + ql.kh)
+// (f16 hi / lo halves, f32 sums; the two small products share an accumulator,
+// which k_prefill_fa64 does not: a rounding 2^-11 of the score's), exp2 of log2-scaled scores with a running
 // maximum, values ph.vh + ph.vl + pl.vh.
 // ---------------------------------------------------------------------------
 constexpr int FT = 32;                // keys per tile

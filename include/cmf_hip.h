@@ -137,8 +137,9 @@ int cmf_gemv_prepared(cmf_weight w, const void* d_planes, const float* d_xs, int
  * operand is prepared into a workspace the library holds in a static device
  * array (1 310 976 B per device, set up by cmf_init), then the GEMV of
  * cmf_gemv_prepared runs on it; the same results as cmf_prep_dev +
- * cmf_gemv_prepared with a caller workspace, bit for bit (one row: the kernel
- * that prepares the row itself, without the workspace).  Weights whose
+ * cmf_gemv_prepared with a caller workspace, bit for bit (one row that y does
+ * not overlap: the kernel that prepares the row itself, without the
+ * workspace).  y may overlap x.  Weights whose
  * operand needs more (cols > 16384) are rejected with an error.  No
  * counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops).  Requires

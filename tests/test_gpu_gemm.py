@@ -1,15 +1,15 @@
 """The large-batch GEMM (batches above 16 rows) and its operand producers at
 the edges of their tiles: row counts that leave part of a 16-row block, a
 wave's 32 / 64 rows or a workgroup, column counts that leave part of a group
-of tiles or of a 64-column chunk, one K part and several, 32 and 64 weight
-rows a wave, and rows that the wave-per-row producer holds or that take the
-general one."""
+of tiles or of a 64-column chunk, one K part and several, 32 weight rows a
+wave (test_gpu_gemm_rules has 64), and rows that the wave-per-row producer
+holds or that take the general one."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-# rows, cols, batch: (q4) one part / split K, 32 and 64 rows a wave; the last
+# rows, cols, batch: (q4) one part / split K; the last
 # two: the most columns the wave-per-row producer holds, and past it
 Q4 = [(1000, 1056, 77), (16, 32, 17), (48, 160, 64), (2064, 512, 1030), (3072, 128, 700), (24, 8192, 33), (8, 8224, 18)]
 Q8 = [(1000, 1056, 77), (16, 48, 17), (40, 100, 65), (272, 1000, 130), (4112, 192, 1100), (24, 8192, 33), (8, 8208, 18)]

@@ -47,7 +47,7 @@ def test_moe_forward_batch_matches_oracle(moe_model):
 
 @pytest.mark.parametrize("spec", [True, False])
 def test_moe_decode_tokens_equal_oracle(moe_model, spec):
-    """prefill (the MoE blocks of the chunk in 16-row batches) + decode"""
+    """prefill (more than 16 rows: the MoE blocks' grouped GEMMs) + decode"""
     sm, g = moe_model
     from cmf_amd import synth
     prompt = synth.ids(34, 40, CFG["vocab"])

@@ -1,7 +1,7 @@
-"""The prefill attention's query blocks (128 rows of a kv head's query heads,
-paired, the longer block's keys in two halves) at their edges: one and two
-query heads a kv head, one row, a row more than a block, odd and even numbers of blocks, one
-KV head per XCD (8 KV heads) and placed by the grid.  The second layer's K / V
+"""The prefill attention's query blocks of contexts up to 576 keys (64 rows of
+a kv head's query heads, paired) at their edges: one and two query heads a kv
+head, one row, a row more than a block or a pair of them, odd and even numbers
+of blocks, one KV head per XCD (8 KV heads) and placed by the grid.  The second layer's K / V
 rows see the first layer's attention at every position, so they are compared
 with the oracle's per-position forwards in 64-row pieces, within the relative
 L2 of 1e-4 that the prefill is held to everywhere (both sides sum in f32, in
@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("heads,kv,n", [
-    (1, 1, 1), (2, 2, 33), (8, 8, 129), (8, 8, 385),     # 128 positions a block
-    (4, 2, 64), (4, 2, 65), (16, 8, 193),                # 64
+    (1, 1, 1), (2, 2, 33), (8, 8, 129), (8, 8, 385),     # 64 positions a block
+    (4, 2, 64), (4, 2, 65), (16, 8, 193),                # 32
     (16, 8, 321), (2, 1, 448),
 ])
 def test_prefill_attention_block_edges(gpu, heads, kv, n):
