@@ -1459,8 +1459,8 @@ int cmf_decode(cmf_model m, int max_tokens, const cmf_sampler_config* sc, uint64
         // which replays a captured round without a host round trip between
         // them, as far as they stay within the 512-position step that the
         // captured round of the next one is sized for: a bound on all of them
-        // would take the fused blocks from rounds that still fit them (context
-        // 2600, 600 tokens, one head model of 28 layers: 544 ms, 526 without).
+        // would take the fused blocks from rounds that still fit them (28
+        // layers of 1024, context 2600, 600 plain tokens: 544 ms, 460 in steps).
         // Rounds under the monitor are timed one by one.  Where the positions
         // would not fit, one at a time up to the same error.  (A k out of range
         // is left to be refused by the round.)
