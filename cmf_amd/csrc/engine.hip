@@ -178,9 +178,21 @@ struct cmf_model_s {
 
 namespace {
 
+// Zeroes device memory, done on return: the clear is ordered on the null
+// stream only, which the library's (non-blocking) streams do not wait for.
+int clear_dev(void* p, size_t bytes) {
+    CMF_HIP(hipMemset(p, 0, bytes));
+    CMF_HIP(hipStreamSynchronize(nullptr));
+    return CMF_OK;
+}
+
 int dalloc(cmf_model_s* m, void** p, size_t bytes) {
     CMF_HIP(hipMalloc(p, bytes));
-    CMF_HIP(hipMemset(*p, 0, bytes));
+    if (clear_dev(*p, bytes) != CMF_OK) {
+        (void)hipFree(*p);
+        *p = nullptr;
+        return CMF_ERR;
+    }
     m->allocs.push_back(*p);
     return CMF_OK;
 }
@@ -588,7 +600,6 @@ int ensure_prefill_bufs(cmf_model_s* m) {
         const size_t cells = prefill_attention_cells((int)R, c.n_heads, c.n_kv);
         if (dalloc(m, &m->pf_part, prefill_attention_scratch((int)R, c.n_heads, c.n_kv)) || dalloc_t(m, &m->pf_mcell, cells))
             return CMF_ERR;
-        CMF_HIP(hipMemset(m->pf_mcell, 0, cells * sizeof(unsigned long long)));
     }
     if (dalloc_t(m, &m->pf_h, R * H) || dalloc_t(m, &m->pf_qkv, R * QKV) ||
         dalloc_t(m, &m->pf_ao, R * c.n_heads * c.head_dim) || dalloc_t(m, &m->pf_gu, R * 2 * c.inter) ||
@@ -597,10 +608,7 @@ int ensure_prefill_bufs(cmf_model_s* m) {
         dalloc(m, (void**)&m->pf_khl, (size_t)c.n_kv * ((c.max_seq + 127) / 128 * 128) * c.head_dim * 8) ||
         dalloc_t(m, &m->pf_cells, PREFILL_XCD_CELLS) || dalloc_t(m, &m->pf_err, 1))
         return CMF_ERR;
-    // (tags start at 1, so the zeroed cells hold none)
-    CMF_HIP(hipMemset(m->pf_cells, 0, PREFILL_XCD_CELLS * sizeof(unsigned long long)));
-    CMF_HIP(hipMemset(m->pf_err, 0, sizeof(int)));
-    return CMF_OK;
+    return CMF_OK;  // (tags start at 1: the zeroed cells hold none)
 }
 
 // Whether l's routed experts run as large-batch GEMMs over cnt prefill rows:
@@ -996,7 +1004,7 @@ static int xl_check(cmf_model m) {
         e |= 1;
     }
     if (e != 0) {
-        CMF_HIP(hipMemset(m->xl.err, 0, sizeof(int)));
+        if (clear_dev(m->xl.err, sizeof(int)) != CMF_OK) return CMF_ERR;
         m->xl_on = false;
         m->xl_fallbacks += 1;
         drop_graph(m);
@@ -1094,7 +1102,7 @@ int cmf_prefill(cmf_model m, const int32_t* ids, int n) {
         perr = 1;
     if (perr && !m->pf_xcd_off) {
         m->pf_xcd_off = true;
-        CMF_HIP(hipMemset(m->pf_err, 0, sizeof(int)));
+        if (clear_dev(m->pf_err, sizeof(int)) != CMF_OK) return CMF_ERR;
         return cmf_prefill(m, ids, n);
     }
     m->next_pos_host = n;
